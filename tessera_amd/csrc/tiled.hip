@@ -5,8 +5,8 @@
 // which on gfx950 is refused today (no tile row for gfx9_5). Same product and
 // fused stages (engine/plan/lower/src/kernels/map.rs:155-185).
 //
-// gfx950 design (bf16 rows and weights take the pipelined kernel further down, which
-// shares the tile order, swizzle and epilogue described here):
+// gfx950 design (depths that are a multiple of 64 take the pipelined kernel further down,
+// which shares the tile, swizzle and epilogue described here):
 //  * 128x128 output tile per 256-thread group (4 waves in 2x2, each 64x64 =
 //    4x4 v_mfma_f32_16x16x32_bf16 tiles), k in 64-deep steps; 64x64 tiles (waves of
 //    32x32) when 128x128 would give fewer than 2 groups per CU, since each group is a
@@ -31,8 +31,8 @@
 
 namespace {
 
-#ifndef TS_PIPE_WIDE
-#define TS_PIPE_WIDE 1
+#ifndef TS_PIPE_SMALL
+#define TS_PIPE_SMALL 256
 #endif
 constexpr int BM = 128, BN = 128, BK = 64;  // the default tile; BT = 64 for products with few tiles
 constexpr int kThreads = 256;
@@ -303,59 +303,95 @@ __global__ __launch_bounds__(kThreads) void tiled_kernel(TiledParams p) {
 
 
 // ---------------------------------------------------------------------------
-// The pipelined form for bf16 rows and weights (k a multiple of 64): TM x TN tiles,
-// 4 waves in 2 x 2 (each (TM/2) x (TN/2)), and NS LDS stages KD deep filled straight
-// from memory with global_load_lds_dwordx4 (no staging registers, no LDS stores),
-// NS - 1 of them in flight ahead of the MFMAs, groups in an XCD-aware order, and
-// each configuration sized so two groups share a CU: one group's loads, barriers and
-// epilogue overlap the other's matrix work. bf16 results leave through LDS as whole
-// rows. The register-staged form above still serves f32 rows and e4m3 weights.
+// The pipelined form (k a multiple of 64): TM x TN tiles, 4 waves, and NS LDS stages KD
+// deep filled straight from memory with global_load_lds_dwordx4 (no staging registers,
+// no LDS stores), NS - 1 of them in flight ahead of the MFMAs, groups in an XCD-aware
+// order, and each configuration sized so two groups share a CU: one group's loads,
+// barriers and epilogue overlap the other's matrix work. bf16 results leave through LDS
+// as whole rows.
+//  * bf16 rows and weights: waves in 2 x 2, each (TM/2) x (TN/2).
+//  * f32 rows (XF32) lie in LDS as f32, as many bytes as the two bf16 parts would take;
+//    a lane splits the 8 values of a fragment into hi = bf16(x), lo = bf16(x - hi) right
+//    after reading them (24 vector instructions a fragment). The waves are stacked along
+//    the rows, so each fragment is split by one wave only, at the same LDS bytes read per
+//    MFMA as 2 x 2 (a row fragment is two reads here, a weight fragment one).
+//  * e4m3 weights (W8) lie in LDS as codes, half the bytes; a lane reads 16 codes of its
+//    weight row and decodes them to the two fragments of a 64-deep step (8 conversions).
+//    The matrix unit sums k in any order, so the rows' fragments are read at the same k.
+// Register-staged against this form: 1000 f32 rows by bf16 weights 4096 x 1024 64.2 -> 27.3
+// us, 1024 x 3072 92.6 -> 28.3 us; 1000 bf16 rows by e4m3 gate/up 2 x 14336 x 4096 560 -> 248
+// us (947 TFLOP/s), down 4096 x 14336 249 -> 159 us. What the register-staged form spent
+// was the load latency of every k step, with no stage in flight behind its barrier. It
+// still serves depths that are no multiple of 64 and the stage chains of picked products.
 // ---------------------------------------------------------------------------
-template <int TM, int TN, int KD, int NS>
-struct Pipe {
-    static constexpr int RB = KD * 2;          // bytes of one LDS row (KD bf16)
-    static constexpr int CPR = KD / 8;         // 16-byte chunks per row
-    static constexpr int RPI = 1024 / RB;      // rows one load instruction fills
-    static constexpr int NA = TM / RPI / 4;    // A load instructions per wave per stage
-    static constexpr int NB = TN / RPI / 4;    // B load instructions per wave per stage
-    static constexpr int A_BYTES = TM * RB, STAGE = (TM + TN) * RB, LDS = NS * STAGE;
-    static constexpr int WM = TM / 2, WN = TN / 2, FI = WM / 16, FJ = WN / 16;
-    static_assert(NA >= 1 && NB >= 1 && (KD == 32 || KD == 64), "pipe shape");
+// A stage's operand rows in LDS: RB bytes a row in 16-byte chunks.
+template <int RB>
+struct Rows {
+    static constexpr int CPR = RB / 16;    // chunks per row
+    static constexpr int RPI = 1024 / RB;  // rows one load instruction fills
+    static_assert(RB == 64 || RB == 128 || RB == 256, "row bytes");
 
-    // Byte offset of logical chunk c of row r. 128-byte rows: chunk c ^ (r & 7) of row
-    // r. 64-byte rows: rows pair up in 128-byte lines L = r / 2, and 16-byte unit
-    // u = 4 (r & 1) + c of a line sits at u ^ (L & 7). Either way the 16 rows one
-    // fragment read touches (one chunk each) spread over all banks (measured: no
-    // conflicts; a per-row XOR of 64-byte rows conflicts).
+    // Byte offset of chunk c of row r. 256- and 128-byte rows: chunk c ^ (r & (CPR - 1)).
+    // 64-byte rows: rows pair up in 128-byte lines L = r / 2, and 16-byte unit u = 4 (r &
+    // 1) + c of a line sits at u ^ (L & 7). Either way the 16 rows one fragment read
+    // touches (one chunk each) spread over all banks (measured: no conflicts; a per-row
+    // XOR of 64-byte rows conflicts).
     TS_DEV static uint32_t at(uint32_t r, uint32_t c) {
-        if (CPR == 8) return r * 128 + ((c ^ (r & 7)) << 4);
+        if (RB >= 128) return r * RB + ((c ^ (r & (CPR - 1))) << 4);
         const uint32_t L = r >> 1, u = (r & 1) * 4 + c;
         return L * 128 + ((u ^ (L & 7)) << 4);
     }
-    // The row (within the RPI rows an instruction fills) and logical chunk that lane l
-    // of a load instruction brings: the lane lands at byte 16 l of the instruction's KiB.
-    TS_DEV static void source(uint32_t l, uint32_t &row, uint32_t &chunk) {
-        const uint32_t line = l >> 3, u = (l & 7) ^ line;  // line & 7 == line: 8 lines per KiB
-        if (CPR == 8) {
-            row = line;
-            chunk = u;
+    // The row and chunk that lane l of load instruction b brings (the lane lands at byte
+    // 16 l of the instruction's KiB, whose first row is RPI b).
+    TS_DEV static void source(uint32_t b, uint32_t l, uint32_t &row, uint32_t &chunk) {
+        if (RB >= 128) {
+            row = RPI * b + l / CPR;
+            chunk = (l % CPR) ^ (row & (CPR - 1));
         } else {
-            row = 2 * line + (u >> 2);
+            const uint32_t line = l >> 3, u = (l & 7) ^ line;  // 8 lines per KiB: line is L & 7
+            row = RPI * b + 2 * line + (u >> 2);
             chunk = u & 3;
         }
     }
 };
 
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8>
+struct Pipe {
+    using A = Rows<KD * (XF32 ? 4 : 2)>;
+    using B = Rows<KD * (W8 ? 1 : 2)>;
+    static constexpr int AE = XF32 ? 4 : 8, BE = W8 ? 16 : 8;  // elements per chunk
+    static constexpr int NA = TM / A::RPI / 4;  // A load instructions per wave per stage
+    static constexpr int NB = TN / B::RPI / 4;  // B load instructions per wave per stage
+    static constexpr int A_BYTES = TM * A::CPR * 16, STAGE = A_BYTES + TN * B::CPR * 16, LDS = NS * STAGE;
+    static constexpr int GM = XF32 ? 4 : 2, GN = 4 / GM;  // waves along the rows and the columns
+    static constexpr int WM = TM / GM, WN = TN / GN, FI = WM / 16, FJ = WN / 16;
+    static_assert(NA >= 1 && NB >= 1 && FI >= 1 && (KD == 64 || (KD == 32 && !W8)), "pipe shape");
+};
+
+// Eight f32 values (two chunks) as the two bf16 parts hi = bf16(x), lo = bf16(x - hi).
+TS_DEV void split_f32(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {
+    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(ts_f32x2{v[2 * e], v[2 * e + 1]}, ts_bf16x2));
+        const ts_f32x2 rest = {v[2 * e] - lo_bf16(h[e]), v[2 * e + 1] - hi_bf16(h[e])};
+        l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, ts_bf16x2));
+    }
+    hi = as_bf16x8(u32x4{h[0], h[1], h[2], h[3]});
+    lo = as_bf16x8(u32x4{l[0], l[1], l[2], l[3]});
+}
+
 constexpr uint32_t kBand = 8;  // tile rows per band of the XCD-aware order
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// Waits until at most N of this wave's loads are outstanding, then meets the group's
-// other waves (no fence: the LDS reads of the previous k-step completed before their
-// MFMAs, and the loads waited for here wrote LDS directly).
+// Waits until at most N of this wave's loads are outstanding and its LDS reads of the
+// previous k-step are back, then meets the group's other waves (the loads waited for here
+// wrote LDS directly).
 template <int N>
 TS_DEV void pipe_wait() {
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // The wait for a stage with `ahead` later stages (L loads each) still allowed in flight.
@@ -375,12 +411,12 @@ TS_DEV const char *uniform_ptr(const void *ptr) {
     return (const char *)(((uint64_t)hi << 32) | lo);
 }
 
-template <int TM, int TN, int KD, int NS, bool SILU, bool PICK, bool CHAIN>
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, bool CHAIN>
 __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) {
-    using P = Pipe<TM, TN, KD, NS>;
+    using P = Pipe<TM, TN, KD, NS, XF32, W8>;
     extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: two groups share a CU
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t wm = wave >> 1, wn = wave & 1;
+    const uint32_t wm = wave / P::GN, wn = wave % P::GN;
     const uint32_t col = lane & 15, grp = lane >> 4;
     constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
     uint32_t tx = blockIdx.x, ty = blockIdx.y;
@@ -399,7 +435,8 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
     }
     uint32_t n0 = tx * OC;
     uint32_t m0 = ty * TM, mend = p.m;
-    const uint16_t *w = (const uint16_t *)p.w;
+    const char *w = (const char *)p.w;
+    const uint16_t *scale = p.w_scale;
     if (PICK) {
         uint32_t y = blockIdx.y;
         if (p.pick_cols) {
@@ -441,56 +478,55 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
         const uint32_t e = lo;
         m0 = p.row_start[e] + (y - p.tile_start[e]) * TM;
         mend = p.row_start[e + 1];
-        w += ((size_t)e * p.stride + p.offset) * p.k;
+        const size_t first_row = (size_t)e * p.stride + p.offset;
+        w += first_row * p.k * (W8 ? 1 : 2);
+        if (W8) scale += first_row;
     }
     // PICK: the output row of tile row tr (~0u past the matrix's rows), read where needed
     // (no LDS copy, so two groups' stages fill a CU's LDS).
     auto row_out = [&](uint32_t tr) { return m0 + tr < mend ? p.perm[m0 + tr] : 0xffffffffu; };
-    // Element offsets (at k = 0) of the row each of this lane's loads reads, and the
-    // logical chunk it fetches: instruction i of the wave fills rows RPI b .. RPI b +
-    // RPI - 1, b = NA wave + i (A) or NB wave + i (B). Rows past the end read a row
-    // that exists (never stored).
-    uint32_t rl, lc;
-    P::source(lane, rl, lc);
+    // Element offsets (at k = 0) of the chunk each of this lane's loads reads: instruction
+    // NA wave + i (A) or NB wave + i (B) of the stage. Rows past the end read a row that
+    // exists (never stored).
     uint32_t aoff[P::NA], boff[P::NB];
 #pragma unroll
     for (int i = 0; i < P::NA; i++) {
-        const uint32_t r = P::RPI * (wave * P::NA + i) + rl;
-        uint32_t xr;
+        uint32_t r, c, xr;
+        P::A::source(wave * P::NA + i, lane, r, c);
         if (PICK) {
             const uint32_t o = row_out(r);
             xr = (o != 0xffffffffu ? o : p.perm[m0]) / p.repeat;
         } else {
             xr = min(m0 + r, p.m - 1);
         }
-        aoff[i] = xr * p.k + lc * 8;
+        aoff[i] = xr * p.k + c * P::AE;
     }
 #pragma unroll
     for (int i = 0; i < P::NB; i++) {
-        const uint32_t r = P::RPI * (wave * P::NB + i) + rl;
-        uint32_t nr;
+        uint32_t r, c, nr;
+        P::B::source(wave * P::NB + i, lane, r, c);
         if (SILU) {
             // Each wave's WN weight rows: WN/2 gate rows, then the up rows of the same columns.
             const uint32_t half = r / P::WN, within = r % P::WN;
-            const uint32_t c = min(n0 + half * (P::WN / 2) + within % (P::WN / 2), p.n - 1);
-            nr = within < P::WN / 2 ? c : p.n + c;
+            const uint32_t col0 = min(n0 + half * (P::WN / 2) + within % (P::WN / 2), p.n - 1);
+            nr = within < P::WN / 2 ? col0 : p.n + col0;
         } else {
             nr = min(n0 + r, p.n - 1);
         }
-        boff[i] = nr * p.k + lc * 8;
+        boff[i] = nr * p.k + c * P::BE;
     }
-    const uint16_t *xs = (const uint16_t *)p.x;
 
     auto fetch = [&](uint32_t slot, uint32_t k0) {
         char *stage = lds + slot * P::STAGE;
-        const char *xb = uniform_ptr(xs + k0), *wb = uniform_ptr(w + k0);
+        const char *xb = uniform_ptr((const char *)p.x + (size_t)k0 * (XF32 ? 4 : 2));
+        const char *wb = uniform_ptr(w + (size_t)k0 * (W8 ? 1 : 2));
 #pragma unroll
         for (int i = 0; i < P::NA; i++)
-            __builtin_amdgcn_global_load_lds((const void *)(xb + (size_t)aoff[i] * 2),
+            __builtin_amdgcn_global_load_lds((const void *)(xb + (size_t)aoff[i] * (XF32 ? 4 : 2)),
                                              (lds_void *)(stage + (wave * P::NA + i) * 1024), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < P::NB; i++)
-            __builtin_amdgcn_global_load_lds((const void *)(wb + (size_t)boff[i] * 2),
+            __builtin_amdgcn_global_load_lds((const void *)(wb + (size_t)boff[i] * (W8 ? 1 : 2)),
                                              (lds_void *)(stage + P::A_BYTES + (wave * P::NB + i) * 1024), 16, 0, 0);
     };
 
@@ -517,21 +553,45 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
         // tile) skip their MFMAs; their loads and the barriers stay, so every wave keeps
         // the same pipeline.
         auto step = [&](const bool all) {
+            u32x4 codes[W8 ? P::FJ : 1];  // e4m3: the 16 codes of a 64-deep step, k 16 grp .. + 15
+            if (W8)
+#pragma unroll
+                for (int j = 0; j < P::FJ; j++)
+                    codes[j] = *(const u32x4 *)(sb + P::B::at(wn * P::WN + j * 16 + col, grp));
 #pragma unroll
             for (int ks = 0; ks < KD / 32; ks++) {
-                const uint32_t chunk = ks * 4 + grp;
-                bf16x8 af[P::FI], bfr[P::FJ];
+                // The 8 k values of this lane: eighth `chunk` of the step (e4m3: the half of its codes).
+                const uint32_t chunk = W8 ? 2 * grp + ks : ks * 4 + grp;
+                bf16x8 af[P::FI], al[XF32 ? P::FI : 1], bfr[P::FJ];
 #pragma unroll
                 for (int i = 0; i < P::FI; i++)
-                    if (all || (uint32_t)i < live_frags)
-                        af[i] = as_bf16x8(*(const u32x4 *)(sa + P::at(wm * P::WM + i * 16 + col, chunk)));
+                    if (all || (uint32_t)i < live_frags) {
+                        const uint32_t r = wm * P::WM + i * 16 + col;
+                        if (XF32)
+                            split_f32(*(const f32x4 *)(sa + P::A::at(r, 2 * chunk)),
+                                      *(const f32x4 *)(sa + P::A::at(r, 2 * chunk + 1)), af[i], al[XF32 ? i : 0]);
+                        else
+                            af[i] = as_bf16x8(*(const u32x4 *)(sa + P::A::at(r, chunk)));
+                    }
 #pragma unroll
-                for (int j = 0; j < P::FJ; j++) bfr[j] = as_bf16x8(*(const u32x4 *)(sb + P::at(wn * P::WN + j * 16 + col, chunk)));
+                for (int j = 0; j < P::FJ; j++) {
+                    if (W8) {
+                        const u32x4 q = codes[W8 ? j : 0];
+                        const u32x2 lo = e4m3x4_to_bf16x4(ks ? q.z : q.x), hi = e4m3x4_to_bf16x4(ks ? q.w : q.y);
+                        bfr[j] = as_bf16x8(u32x4{lo.x, lo.y, hi.x, hi.y});
+                    } else {
+                        bfr[j] = as_bf16x8(*(const u32x4 *)(sb + P::B::at(wn * P::WN + j * 16 + col, chunk)));
+                    }
+                }
 #pragma unroll
                 for (int i = 0; i < P::FI; i++)
-                    if (all || (uint32_t)i < live_frags)
+                    if (all || (uint32_t)i < live_frags) {
 #pragma unroll
                         for (int j = 0; j < P::FJ; j++) acc[i][j] = mfma16(bfr[j], af[i], acc[i][j]);
+                        if (XF32)
+#pragma unroll
+                            for (int j = 0; j < P::FJ; j++) acc[i][j] = mfma16(bfr[j], al[XF32 ? i : 0], acc[i][j]);
+                    }
             }
         };
         if (!PICK || live_frags >= (uint32_t)P::FI) step(true);
@@ -542,13 +602,28 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
     // wm WM + 16 i + col and columns wn WN + 16 j + 4 grp .. + 3 (SILU: gate in j < FJ/2,
     // up in j + FJ/2, output columns wn WN/2 + 16 j + 4 grp .. + 3).
     const uint32_t N = p.n;
-    auto value = [&](int i, int j, int r) {
-        const float g = acc[i][j][r];
-        const float u = SILU ? acc[i][j + P::FJ / 2][r] : 0.0f;
-        return SILU ? (p.pair_sum ? g + u : g / (1.0f + expf(-g)) * u) : g;
-    };
     constexpr int JO = SILU ? P::FJ / 2 : P::FJ;
     constexpr uint32_t WO = SILU ? P::WN / 2 : P::WN;
+    // e4m3: each weight row's scale on its finished sums.
+    if (W8) {
+#pragma unroll
+        for (int j = 0; j < JO; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t n = min(n0 + wn * WO + j * 16 + 4 * grp + r, N - 1);
+                const float sg = bf16_float(scale[n]), su = SILU ? bf16_float(scale[N + n]) : 0.0f;
+#pragma unroll
+                for (int i = 0; i < P::FI; i++) {
+                    acc[i][j][r] *= sg;
+                    if (SILU) acc[i][j + JO][r] *= su;
+                }
+            }
+    }
+    auto value = [&](int i, int j, int r) {
+        const float g = acc[i][j][r];
+        const float u = SILU ? acc[i][j + (SILU ? P::FJ / 2 : 0)][r] : 0.0f;
+        return SILU ? (p.pair_sum ? g + u : g / (1.0f + expf(-g)) * u) : g;
+    };
     if (!PICK && p.out_bf16 && !(p.stages & TS_AFTER_ADD) && !p.after.count) {
         // bf16 rows through LDS: the tile as TM rows of OC bf16 (16-byte chunks
         // XOR-swizzled by row), then whole 16-byte chunks of rows to memory.
@@ -638,22 +713,19 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
     }
 }
 
-template <int TM, int TN, int KD, int NS, bool PICK>
+// CHAIN: the instance that runs stage chains (64 x 64 tiles only: larger ones would spill).
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool PICK, bool CHAIN = false>
 int pipe_launch(TiledParams p, bool silu, void *stream) {
-    constexpr int lds = Pipe<TM, TN, KD, NS>::LDS;
-    const void *kerns[4] = {(const void *)tiled_pipe_kernel<TM, TN, KD, NS, false, PICK, false>,
-                            (const void *)tiled_pipe_kernel<TM, TN, KD, NS, true, PICK, false>,
-                            (const void *)tiled_pipe_kernel<TM, TN, KD, NS, false, PICK, true>,
-                            (const void *)tiled_pipe_kernel<TM, TN, KD, NS, true, PICK, true>};
+    constexpr int lds = Pipe<TM, TN, KD, NS, XF32, W8>::LDS;
+    const void *k = silu ? (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, CHAIN>
+                         : (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, CHAIN>;
     // The dynamic LDS size is raised once per kernel (thread-safe static initialisation).
-    static const hipError_t attr[4] = {
-        hipFuncSetAttribute(kerns[0], hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-        hipFuncSetAttribute(kerns[1], hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-        hipFuncSetAttribute(kerns[2], hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-        hipFuncSetAttribute(kerns[3], hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
-    const int which = (silu ? 1 : 0) + (p.after.count ? 2 : 0);
-    if (attr[which]) return ts::hip_status(attr[which], "tiled (pipelined): LDS attribute");
-    const void *k = kerns[which];
+    static const hipError_t attr[2] = {
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, CHAIN>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, CHAIN>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
+    if (attr[silu]) return ts::hip_status(attr[silu], "tiled (pipelined): LDS attribute");
     const uint32_t oc = silu ? TN / 2 : TN;
     const uint32_t gx = (p.n + oc - 1) / oc;
     dim3 grid;
@@ -682,11 +754,27 @@ int pipe_launch(TiledParams p, bool silu, void *stream) {
     return TS_OK;
 }
 
-// The pipelined kernels take bf16 operands, whole 64-deep k steps and element offsets
-// of rows (x rows, and the rows of one weight matrix) that fit 32 bits.
-bool pipe_fits(int x_dtype, int w_dtype, uint32_t x_rows, uint32_t k, uint32_t w_rows) {
-    return x_dtype == TS_BF16 && w_dtype == TS_BF16 && k % 64 == 0 && (uint64_t)x_rows * k < (1ull << 32) &&
-           (uint64_t)w_rows * k < (1ull << 32);
+// The pipelined kernels take whole 64-deep k steps and element offsets of rows (x rows,
+// and the rows of one weight matrix) that fit 32 bits.
+bool pipe_fits(uint32_t x_rows, uint32_t k, uint32_t w_rows) {
+    return k % 64 == 0 && (uint64_t)x_rows * k < (1ull << 32) && (uint64_t)w_rows * k < (1ull << 32);
+}
+
+// 64 x 64 tiles, four stages of 16 KiB or three of 20 to 24.
+template <bool CHAIN>
+int pipe_small(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
+    if (xf) return w8 ? pipe_launch<64, 64, 64, 3, true, true, false, CHAIN>(p, silu, stream)
+                      : pipe_launch<64, 64, 64, 3, true, false, false, CHAIN>(p, silu, stream);
+    return w8 ? pipe_launch<64, 64, 64, 4, false, true, false, CHAIN>(p, silu, stream)
+              : pipe_launch<64, 64, 64, 4, false, false, false, CHAIN>(p, silu, stream);
+}
+
+// 128 x 128 tiles of f32 rows or e4m3 weights.
+template <bool PICK>
+int pipe_wide(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
+    if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK>(p, silu, stream)
+                      : pipe_launch<128, 128, 32, 3, true, false, PICK>(p, silu, stream);
+    return pipe_launch<128, 128, 64, 3, false, true, PICK>(p, silu, stream);
 }
 
 using Kern = void (*)(TiledParams);
@@ -745,7 +833,8 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
     TS_REQUIRE(gy <= 65535, "tiled: m=%u too large for one launch", a->m);
     p.perm = p.row_start = p.tile_start = nullptr;
     p.matrices = 0; p.repeat = 1; p.stride = 0; p.offset = 0;
-    if (pipe_fits(a->x_dtype, w_dtype, a->m, a->k, silu ? 2 * a->n : a->n)) {
+    const bool xf = a->x_dtype == TS_F32, w8 = w_dtype == TS_E4M3;
+    if (pipe_fits(a->m, a->k, silu ? 2 * a->n : a->n)) {
         // 128 x 128 tiles from one tile per CU up (fewer, larger tiles read less per
         // flop), 64 x 64 below that (measured on the 2048-row projections: q with 256
         // tiles of 128 runs 1.15x faster than with 1024 of 64; o, kv and down with 128
@@ -758,15 +847,14 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
         const uint64_t tiles192 = (a->n + oc * 3 / 2 - 1) / (oc * 3 / 2) * ((a->m + 127) / 128);
         const bool wide = ((tiles192 + 511) / 512) * 3 < ((tiles + 511) / 512) * 2;
         // A stage chain takes 64 x 64 tiles: at 128 x 128 its values and sums spill.
-        if (tiles >= 256 && !p.after.count) {
-            if (wide && TS_PIPE_WIDE) return pipe_launch<128, 192, 64, 2, false>(p, silu, stream);
-            return pipe_launch<128, 128, 64, 2, false>(p, silu, stream);
-        }
-        return pipe_launch<64, 64, 64, 4, false>(p, silu, stream);
+        if (p.after.count) return pipe_small<true>(p, xf, w8, silu, stream);
+        if (tiles < TS_PIPE_SMALL) return pipe_small<false>(p, xf, w8, silu, stream);
+        if (xf || w8) return pipe_wide<false>(p, xf, w8, silu, stream);
+        if (wide) return pipe_launch<128, 192, 64, 2, false, false, false>(p, silu, stream);
+        return pipe_launch<128, 128, 64, 2, false, false, false>(p, silu, stream);
     }
     const bool chain = p.after.count;
-    Kern k = bt == 64 ? pick_kernel<64, false>(a->x_dtype == TS_F32, w_dtype == TS_E4M3, silu, chain)
-                      : pick_kernel<128, false>(a->x_dtype == TS_F32, w_dtype == TS_E4M3, silu, chain);
+    Kern k = bt == 64 ? pick_kernel<64, false>(xf, w8, silu, chain) : pick_kernel<128, false>(xf, w8, silu, chain);
     hipLaunchKernelGGL(k, dim3(gx, gy), dim3(kThreads), 0, (hipStream_t)stream, p);
     TS_CHECK_LAUNCH("tiled launch");
     return TS_OK;
@@ -826,11 +914,14 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // A stage chain takes the register-staged kernel (the pipelined one's chain variant spills).
     // 128 x 192 tiles where the columns divide evenly (fewer re-reads of the gathered
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
-    if (pipe_fits(a->x_dtype, a->w_dtype, a->rows, a->k, a->stride) && !p.after.count) {
-        if ((silu ? a->n % 96 : a->n % 192) == 0) return pipe_launch<128, 192, 64, 2, true>(p, silu, stream);
-        return pipe_launch<128, 128, 64, 2, true>(p, silu, stream);
+    const bool xf = a->x_dtype == TS_F32, w8 = a->w_dtype == TS_E4M3;
+    if (pipe_fits(a->rows, a->k, a->stride) && !p.after.count) {
+        if (xf || w8) return pipe_wide<true>(p, xf, w8, silu, stream);
+        if ((silu ? a->n % 96 : a->n % 192) == 0)
+            return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);
+        return pipe_launch<128, 128, 64, 2, false, false, true>(p, silu, stream);
     }
-    Kern k = pick_kernel<BM, true>(a->x_dtype == TS_F32, a->w_dtype == TS_E4M3, silu, p.after.count != 0);
+    Kern k = pick_kernel<BM, true>(xf, w8, silu, p.after.count != 0);
     hipLaunchKernelGGL(k, dim3(gx, gy), dim3(kThreads), 0, (hipStream_t)stream, p);
     TS_CHECK_LAUNCH("picked launch");
     return TS_OK;

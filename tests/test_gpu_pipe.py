@@ -1,0 +1,103 @@
+"""The pipelined tiles over every operand form (f32 or bf16 rows, bf16 or e4m3 weights)
+at the edges of their tiles, against the oracle's product within product_bound."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tests.helpers import bf16_bits_normal, from_dev, linear_bound, max_rel, rng, to_dev
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+FORMS = [("f32", "bf16"), ("f32", "e4m3"), ("bf16", "e4m3")]
+
+
+def operands(r, m, rows, k, x, w):
+    """(device operands and scale, the f32 values of x and w, the oracle's product)."""
+    if x == "f32":
+        xd = xf = r.standard_normal((m, k)).astype(np.float32)
+    else:
+        xd, xf = bf16_bits_normal(r, (m, k))
+    if w == "bf16":
+        wd, wf = bf16_bits_normal(r, (rows, k), 0.05)
+        return to_dev(xd, torch), to_dev(wd, torch), None, xf, wf, O.product_bf16w(xf, wd)
+    v = (r.standard_normal((rows, k)) * 0.05).astype(np.float32)
+    s = O.bf16_narrow((np.abs(v).max(1) / 448.0).astype(np.float32))
+    codes = O.e4m3_narrow(v / O.bf16_widen(s)[:, None])
+    wf = O.e4m3_widen(codes) * O.bf16_widen(s)[:, None]
+    return (to_dev(xd, torch), to_dev(codes, torch), to_dev(s, torch), xf, wf, O.product_e4m3w(xf, codes, s))
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("m,n,k", [(65, 64, 64), (129, 190, 128), (200, 33, 1024), (1000, 4100, 192),
+                                   (1025, 4096, 64)])
+def test_pipe_edges(m, n, k, x, w):
+    """One k step and several, ragged rows and columns, 64 x 64 tiles (the first three) and
+    128 x 128 ones; with a residual, to f32 and to bf16."""
+    from tessera_amd import rules as R
+    print(f"pipe {x} {w} m={m} n={n} k={k}", flush=True)
+    r = rng(m + n + k)
+    O.set_threads(O.lib().or_threads_available())
+    xd, wd, sd, xf, wf, want = operands(r, m, n, k, x, w)
+    O.set_threads(1)
+    res = r.standard_normal((m, n)).astype(np.float32)
+    got = from_dev(R.linear(xd, wd, w_scale=sd, a0=to_dev(res, torch)))
+    bound = linear_bound(xf, wf)
+    assert np.all(np.abs(got.astype(np.float64) - (want + res)) <= bound + 1e-6)
+    got32 = from_dev(R.linear(xd, wd, w_scale=sd))
+    assert np.all(np.abs(got32.astype(np.float64) - want) <= bound)
+    # The bf16 output (through LDS) is the f32 one rounded once, element for element.
+    got16 = from_dev(R.linear(xd, wd, w_scale=sd, out_dtype=torch.bfloat16))
+    assert np.array_equal(got16, O.bf16_widen(O.bf16_narrow(got32)))
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("m,n,k", [(70, 40, 128), (1030, 2050, 64)])
+def test_pipe_gate_up(m, n, k, x, w):
+    """Gate/up pairs on 64 x 64 and on 128 x 128 tiles: silu(g) u, first-order error of the
+    pair's bounds."""
+    from tessera_amd import rules as R
+    r = rng(m + n + k + 1)
+    O.set_threads(O.lib().or_threads_available())
+    xd, wd, sd, xf, wf, gu = operands(r, m, 2 * n, k, x, w)
+    O.set_threads(1)
+    g, u = gu[:, :n], gu[:, n:]
+    want = O.act("silu", g) * u
+    got = from_dev(R.linear(xd, wd, w_scale=sd, silu_mul=True))
+    b = linear_bound(xf, wf)
+    assert np.all(np.abs(got.astype(np.float64) - want) <= 1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5)
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("silu", [False, True])
+def test_pipe_picked(x, w, silu):
+    """Expert products on the same tiles: matrices of 0, 1, 128, 129 and more rows, ids
+    outside the set."""
+    from tessera_amd import rules as R
+    r = rng(17 + silu)
+    count, n, k, offset = 6, 72, 128, 3
+    used = 2 * n if silu else n
+    stride = used + 5
+    ids = np.concatenate([np.full(c, e) for e, c in ((0, 1), (1, 128), (2, 129), (4, 300), (5, 17), (9, 6))])
+    ids = r.permutation(ids).astype(np.uint32)
+    rows = len(ids)
+    xd, wd, sd, xf, wf, _ = operands(r, rows, count * stride, k, x, w)
+    shape = (count, stride, k)
+    got = from_dev(R.picked(xd, wd.view(shape), to_dev(ids.astype(np.int32), torch), n=n, offset=offset, silu_mul=silu,
+                            w_scale=None if sd is None else sd.view(count, stride)))
+    table = wf.reshape(shape)
+    for e in range(10):
+        sel = ids == e
+        if e >= count:
+            assert np.all(got[sel] == 0.0)
+            continue
+        if not sel.any():
+            continue
+        we = table[e, offset:offset + used]
+        full, b = xf[sel].astype(np.float64) @ we.T.astype(np.float64), linear_bound(xf[sel], we)
+        if not silu:
+            assert np.all(np.abs(got[sel] - full) <= b), f"matrix {e}"
+            continue
+        g, u = full[:, :n], full[:, n:]
+        want = g / (1 + np.exp(-g)) * u
+        assert np.all(np.abs(got[sel] - want) <= 1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5), f"matrix {e}"
