@@ -1,5 +1,5 @@
-// Block-form weights on the matrix unit: the product of many rows (m > 4) against
-// any of the seven block forms.
+// Block-form weights on the matrix unit: the product of many rows (m > 64; blocklanes.hip
+// takes 5..64) against any of the seven block forms.
 //
 // Replaces the reference's tiled and lanes rules reading a block form through its
 // load (engine/rules/linear/src/tiled.rs:297-316, every form of

@@ -109,12 +109,6 @@ TS_DEV uint32_t x_piece(int j, uint32_t g) {
 
 TS_DEV float silu(float v) { return v / (1.0f + expf(-v)); }
 
-// The split sums leave the kernel as agent-scope (write-through) stores: lanes_finish
-// reads them from memory anyway, and lines left dirty in the XCDs' L2s cost a write-
-// back at the kernel's end (plain stores measured 15.1 against 12.9 us on 4096 x 4096
-// e4m3 at m 64).
-TS_DEV void put_part(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
 // One 128-deep chunk of x rows [0, M) in flight: thread t holds pieces i = t + 256 j
 // (piece = 8 k values of one row; 16 pieces per row). Loaded early into registers,
 // written to LDS later (store_x), so the load latency hides under the MFMAs.
@@ -439,7 +433,8 @@ int check(const ts_linear_args *a) {
 
 extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
     if (a && (a->stages & TS_AFTER_ARGMAX)) return (size_t)a->m * 8;  // the keys
-    if (!a || a->m <= 4 || a->m > 64 || ts::block_form(a->w_dtype)) return 0;
+    if (!a || a->m <= 4 || a->m > 64) return 0;
+    if (ts::block_form(a->w_dtype)) return ts::block_lanes_workspace(a);
     const Plan pl = plan(a);
     if (pl.splits <= 1) return 0;
     const size_t per = (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1);
@@ -447,8 +442,11 @@ extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
 }
 
 extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
-    if (a && ts::block_form(a->w_dtype))
-        return a->m <= 4 ? ts::block_gemv_launch(a, stream) : ts::block_tiled_launch(a, stream);
+    if (a && ts::block_form(a->w_dtype)) {
+        if (a->m <= 4) return ts::block_gemv_launch(a, stream);
+        const int few = ts::block_lanes_launch(a, stream);
+        return few != 1 ? few : ts::block_tiled_launch(a, stream);
+    }
     int rc = check(a);
     if (rc) return rc;
     if (a->m <= 4) {

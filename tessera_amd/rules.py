@@ -121,7 +121,10 @@ def _linear(fn: str, x, w, *, out=None, out_dtype=torch.float32, w_scale=None, g
         a.after = C.addressof(after)
     lib = abi.load()
     need = getattr(lib, fn + "_workspace")(C.byref(a)) if hasattr(lib, fn + "_workspace") else 0
-    a.workspace, a.workspace_bytes = workspace(x.device).get(need)
+    # The split sums' scratch is the call's own (the allocator's cache keeps it in stream
+    # order), so products on several streams or threads do not share it.
+    scratch = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    a.workspace, a.workspace_bytes = _ptr(scratch), need
     abi.call(fn, C.byref(a), _stream())
     return out
 
