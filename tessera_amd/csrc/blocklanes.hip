@@ -77,8 +77,6 @@ struct Shape {
     static_assert(LDS <= kMaxLds, "LDS");
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 // Four codes' bytes at byte `at` (a lane's) of a row's words.
 TS_DEV uint32_t word_at(const uint32_t *row, uint32_t at) {
     const uint32_t w = at >> 2;
@@ -222,7 +220,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         char *slot = ring + (step % P::RING) * P::SLOT;
 #pragma unroll
         for (int i = 0; i < P::LOADS; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_void *)(slot + i * 256), 4, woff[i], at, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (ts_lds *)(slot + i * 256), 4, woff[i], at, 0, 0);
     };
 
     // x pieces of a step: piece = t + 512 j: row piece / (4 QS), eighth c of the step's k:

@@ -231,6 +231,24 @@ TS_DEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" :::
 // (plain stores measured 15.1 against 12.9 us on 4096 x 4096 e4m3 at 64 rows).
 TS_DEV void put_part(float *p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+// A raw buffer of 32-bit data from `base` (wave-uniform) up, its bounds left to the caller's
+// offsets.
+TS_DEV __amdgpu_buffer_rsrc_t raw_buffer(const void *base) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+}
+
+// 16 bytes a lane from `buf` (byte offsets `at`, a lane's, and `from`, wave-uniform) straight to
+// LDS: the lane lands at `lds` + 16 lane. A buffer load, not a global one: with a
+// global_load_lds in flight the compiler waits for every load and every LDS read before it
+// uses one, and here LDS reads should return under the matrix work. (The host pass refuses
+// the 16-byte size of gfx950, and would drop the whole kernel.)
+typedef __attribute__((address_space(3))) void ts_lds;
+TS_DEV void buffer_to_lds16(__amdgpu_buffer_rsrc_t buf, void *lds, uint32_t at, uint32_t from) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (ts_lds *)lds, 16, at, from, 0, 0);
+#endif
+}
+
 TS_DEV bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 // In-kernel marks (the reference's TS_MARK ledger, engine/plan/run/src/marks.cuh):

@@ -27,6 +27,8 @@
 //    three), e4m3 weights decode to bf16 on the way into LDS with the per-row
 //    scale applied to the finished sum; SiLU-gate pairs are laid out so a lane
 //    holds gate and up of the same column.
+#include <algorithm>
+
 #include "after.h"
 
 namespace {
@@ -318,9 +320,12 @@ __global__ __launch_bounds__(kThreads) void tiled_kernel(TiledParams p) {
 //  * e4m3 weights (W8) lie in LDS as codes, half the bytes; a lane reads 16 codes of its
 //    weight row and decodes them to the two fragments of a 64-deep step (8 conversions).
 //    The matrix unit sums k in any order, so the rows' fragments are read at the same k.
-// Register-staged against this form: 1000 f32 rows by bf16 weights 4096 x 1024 64.2 -> 27.3
-// us, 1024 x 3072 92.6 -> 28.3 us; 1000 bf16 rows by e4m3 gate/up 2 x 14336 x 4096 560 -> 248
-// us (947 TFLOP/s), down 4096 x 14336 249 -> 159 us. What the register-staged form spent
+//  * The stages come by buffer loads (buffer_to_lds16): with global loads to LDS in flight
+//    the compiler waited for all LDS reads of a step before its first MFMA. With them, and
+//    the steps that refill a stage in a loop without tests: e4m3 4096 x 14336 159 -> 117 us.
+// Register-staged against this form: 1000 f32 rows by bf16 weights 4096 x 1024 64.2 -> 24.7
+// us, 1024 x 3072 92.6 -> 24.9 us; 1000 bf16 rows by e4m3 gate/up 2 x 14336 x 4096 560 -> 223
+// us (1052 TFLOP/s), down 4096 x 14336 249 -> 117 us. What the register-staged form spent
 // was the load latency of every k step, with no stage in flight behind its barrier. It
 // still serves depths that are no multiple of 64 and the stage chains of picked products.
 // ---------------------------------------------------------------------------
@@ -384,8 +389,6 @@ TS_DEV void split_f32(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {
 
 constexpr uint32_t kBand = 8;  // tile rows per band of the XCD-aware order
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 // Waits until at most N of this wave's loads are outstanding and its LDS reads of the
 // previous k-step are back, then meets the group's other waves (the loads waited for here
 // wrote LDS directly).
@@ -405,17 +408,11 @@ TS_DEV void pipe_wait_ahead(uint32_t ahead) {
     }
 }
 
-TS_DEV const char *uniform_ptr(const void *ptr) {
-    const uint64_t v = (uint64_t)ptr;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const char *)(((uint64_t)hi << 32) | lo);
-}
-
 template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, bool CHAIN>
-__global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tiled_pipe_kernel(TiledParams p) {
     using P = Pipe<TM, TN, KD, NS, XF32, W8>;
     extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: two groups share a CU
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wm = wave / P::GN, wn = wave % P::GN;
     const uint32_t col = lane & 15, grp = lane >> 4;
     constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
@@ -485,10 +482,13 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
     // PICK: the output row of tile row tr (~0u past the matrix's rows), read where needed
     // (no LDS copy, so two groups' stages fill a CU's LDS).
     auto row_out = [&](uint32_t tr) { return m0 + tr < mend ? p.perm[m0 + tr] : 0xffffffffu; };
-    // Element offsets (at k = 0) of the chunk each of this lane's loads reads: instruction
-    // NA wave + i (A) or NB wave + i (B) of the stage. Rows past the end read a row that
-    // exists (never stored).
+    // Byte offsets (at k = 0) of the chunk each of this lane's loads reads: instruction NA
+    // wave + i (A) or NB wave + i (B) of the stage, from the tile's first row (A of picked
+    // products: from the first row of x; B of the up rows: from the tile's first up row).
+    // Rows past the end read a row that exists (never stored).
+    constexpr uint32_t XB = XF32 ? 4 : 2, WB = W8 ? 1 : 2;
     uint32_t aoff[P::NA], boff[P::NB];
+    bool up[P::NB];  // wave-uniform: an instruction's rows are all gate or all up rows
 #pragma unroll
     for (int i = 0; i < P::NA; i++) {
         uint32_t r, c, xr;
@@ -497,37 +497,39 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
             const uint32_t o = row_out(r);
             xr = (o != 0xffffffffu ? o : p.perm[m0]) / p.repeat;
         } else {
-            xr = min(m0 + r, p.m - 1);
+            xr = min(r, p.m - 1 - m0);
         }
-        aoff[i] = xr * p.k + c * P::AE;
+        aoff[i] = (xr * p.k + c * P::AE) * XB;
     }
 #pragma unroll
     for (int i = 0; i < P::NB; i++) {
         uint32_t r, c, nr;
         P::B::source(wave * P::NB + i, lane, r, c);
+        up[i] = false;
         if (SILU) {
             // Each wave's WN weight rows: WN/2 gate rows, then the up rows of the same columns.
+            static_assert(!SILU || P::WN / 2 % P::B::RPI == 0, "a load's rows are of one kind");
             const uint32_t half = r / P::WN, within = r % P::WN;
-            const uint32_t col0 = min(n0 + half * (P::WN / 2) + within % (P::WN / 2), p.n - 1);
-            nr = within < P::WN / 2 ? col0 : p.n + col0;
+            nr = min(half * (P::WN / 2) + within % (P::WN / 2), p.n - 1 - n0);
+            up[i] = (wave * P::NB + i) * P::B::RPI % P::WN >= P::WN / 2;
         } else {
-            nr = min(n0 + r, p.n - 1);
+            nr = min(r, p.n - 1 - n0);
         }
-        boff[i] = nr * p.k + c * P::BE;
+        boff[i] = (nr * p.k + c * P::BE) * WB;
     }
 
+    const char *xbase = (const char *)p.x + (PICK ? 0 : (size_t)m0 * p.k * XB);
+    const char *wbase = w + (size_t)n0 * p.k * WB;
+    const __amdgpu_buffer_rsrc_t xbuf = raw_buffer(xbase), wbuf = raw_buffer(wbase),
+                                 ubuf = raw_buffer(wbase + (SILU ? (size_t)p.n * p.k * WB : 0));
     auto fetch = [&](uint32_t slot, uint32_t k0) {
         char *stage = lds + slot * P::STAGE;
-        const char *xb = uniform_ptr((const char *)p.x + (size_t)k0 * (XF32 ? 4 : 2));
-        const char *wb = uniform_ptr(w + (size_t)k0 * (W8 ? 1 : 2));
 #pragma unroll
         for (int i = 0; i < P::NA; i++)
-            __builtin_amdgcn_global_load_lds((const void *)(xb + (size_t)aoff[i] * (XF32 ? 4 : 2)),
-                                             (lds_void *)(stage + (wave * P::NA + i) * 1024), 16, 0, 0);
+            buffer_to_lds16(xbuf, stage + (wave * P::NA + i) * 1024, aoff[i], k0 * XB);
 #pragma unroll
         for (int i = 0; i < P::NB; i++)
-            __builtin_amdgcn_global_load_lds((const void *)(wb + (size_t)boff[i] * (W8 ? 1 : 2)),
-                                             (lds_void *)(stage + P::A_BYTES + (wave * P::NB + i) * 1024), 16, 0, 0);
+            buffer_to_lds16(up[i] ? ubuf : wbuf, stage + P::A_BYTES + (wave * P::NB + i) * 1024, boff[i], k0 * WB);
     };
 
     f32x4 acc[P::FI][P::FJ];
@@ -543,12 +545,9 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
 #pragma unroll
     for (int s = 0; s < NS - 1; s++)
         if ((uint32_t)s < steps) fetch(s, s * KD);
-    for (uint32_t s = 0; s < steps; s++) {
-        // Stage s has landed once no more than the later stages' loads are
-        // outstanding; the barrier also ends every wave's reads of the stage refilled next.
-        pipe_wait_ahead<P::NA + P::NB, NS - 2>(min(steps - 1 - s, (uint32_t)NS - 2));
-        if (s + NS - 1 < steps) fetch((s + NS - 1) % NS, (s + NS - 1) * KD);
-        const char *sa = lds + (s % NS) * P::STAGE, *sb = sa + P::A_BYTES;
+    // The matrix work of the stage in slot `at`.
+    auto multiply = [&](uint32_t at) {
+        const char *sa = lds + at * P::STAGE, *sb = sa + P::A_BYTES;
         // PICK mode: row fragments wholly past the matrix's last row (its partial last
         // tile) skip their MFMAs; their loads and the barriers stay, so every wave keeps
         // the same pipeline.
@@ -596,6 +595,22 @@ __global__ __launch_bounds__(kThreads, 2) void tiled_pipe_kernel(TiledParams p) 
         };
         if (!PICK || live_frags >= (uint32_t)P::FI) step(true);
         else step(false);
+    };
+    // Stage s has landed once no more than the later stages' loads are outstanding; the
+    // barrier also ends every wave's reads of the stage refilled next. The steps that refill
+    // run without a test of what is left.
+    uint32_t s = 0, at = 0, fill = NS - 1;  // the slots of this step and of the stage loaded in it
+    for (; s + NS - 1 < steps; s++) {
+        pipe_wait<(P::NA + P::NB) * (NS - 2)>();
+        fetch(fill, (s + NS - 1) * KD);
+        multiply(at);
+        at = at == NS - 1 ? 0 : at + 1;
+        fill = fill == NS - 1 ? 0 : fill + 1;
+    }
+    for (; s < steps; s++) {
+        pipe_wait_ahead<P::NA + P::NB, NS - 2>(steps - 1 - s);
+        multiply(at);
+        at = at == NS - 1 ? 0 : at + 1;
     }
 
     // Epilogue. acc[i][j] is the transposed 16x16 tile: lane (col, grp) holds tile row
@@ -754,10 +769,10 @@ int pipe_launch(TiledParams p, bool silu, void *stream) {
     return TS_OK;
 }
 
-// The pipelined kernels take whole 64-deep k steps and element offsets of rows (x rows,
-// and the rows of one weight matrix) that fit 32 bits.
-bool pipe_fits(uint32_t x_rows, uint32_t k, uint32_t w_rows) {
-    return k % 64 == 0 && (uint64_t)x_rows * k < (1ull << 32) && (uint64_t)w_rows * k < (1ull << 32);
+// The pipelined kernels take whole 64-deep k steps and byte offsets within the rows a tile
+// may read (256 of x and of w; all of x in picked products) that fit 32 bits.
+bool pipe_fits(uint32_t x_rows, uint32_t k, uint32_t x_bytes) {
+    return k % 64 == 0 && (uint64_t)std::max(x_rows, 256u) * k * x_bytes < (1ull << 32);
 }
 
 // 64 x 64 tiles, four stages of 16 KiB or three of 20 to 24.
@@ -834,7 +849,7 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
     p.perm = p.row_start = p.tile_start = nullptr;
     p.matrices = 0; p.repeat = 1; p.stride = 0; p.offset = 0;
     const bool xf = a->x_dtype == TS_F32, w8 = w_dtype == TS_E4M3;
-    if (pipe_fits(a->m, a->k, silu ? 2 * a->n : a->n)) {
+    if (pipe_fits(0, a->k, 4)) {
         // 128 x 128 tiles from one tile per CU up (fewer, larger tiles read less per
         // flop), 64 x 64 below that (measured on the 2048-row projections: q with 256
         // tiles of 128 runs 1.15x faster than with 1024 of 64; o, kv and down with 128
@@ -915,7 +930,7 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // 128 x 192 tiles where the columns divide evenly (fewer re-reads of the gathered
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
     const bool xf = a->x_dtype == TS_F32, w8 = a->w_dtype == TS_E4M3;
-    if (pipe_fits(a->rows, a->k, a->stride) && !p.after.count) {
+    if (pipe_fits((a->rows - 1) / a->repeat + 1, a->k, xf ? 4 : 2) && !p.after.count) {
         if (xf || w8) return pipe_wide<true>(p, xf, w8, silu, stream);
         if ((silu ? a->n % 96 : a->n % 192) == 0)
             return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);
