@@ -1,4 +1,4 @@
-// Block-form weights on the matrix unit: the product of many rows (m > 64; blocklanes.hip
+// Block-form weights on the matrix unit: the product of many rows (m > 64; stream.hip
 // takes 5..64) against any of the seven block forms.
 //
 // Replaces the reference's tiled and lanes rules reading a block form through its

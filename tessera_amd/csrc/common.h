@@ -47,7 +47,7 @@ int gemv_launch(const ts_linear_args *a, void *stream);
 
 // Block-form weights (TS_Q8_0 .. TS_INT4_G128): codes a block, bytes a block, head
 // bytes (blocks.hip); the m <= 4 decode product (blocks.hip) and the matrix-unit
-// products for more rows (blocklanes.hip, blockmat.hip), each checking its own arguments.
+// products for more rows (stream.hip, blockmat.hip), each checking its own arguments.
 struct BlockShape {
     uint32_t block, bytes, head;
 };
@@ -56,9 +56,12 @@ BlockShape block_shape(int32_t dtype);
 int block_check(const ts_linear_args *a, const char *rule);
 int block_gemv_launch(const ts_linear_args *a, void *stream);
 int block_tiled_launch(const ts_linear_args *a, void *stream);
-// 5..64 rows (blocklanes.hip): 1 when it does not apply; k is split only with the workspace.
-int block_lanes_launch(const ts_linear_args *a, void *stream);
-size_t block_lanes_workspace(const ts_linear_args *a);
+
+// 5..64 rows, weights streamed (stream.hip), arguments already checked: whether a product is
+// for it, the workspace its k split takes (without it k is not split), and the launch.
+bool stream_fits(const ts_linear_args *a);
+size_t stream_workspace(const ts_linear_args *a);
+int stream_launch(const ts_linear_args *a, void *stream);
 
 // Raw sums of a product whose k is split across groups: part[split][gate, up or one][m][n],
 // 16-byte aligned, added in split order and finished (finish.hip).
@@ -66,9 +69,11 @@ struct SplitSum {
     const float *part;
     const uint16_t *w_scale;  // per weight row, or NULL
     const float *head;        // a factor of every sum, or NULL
+    const float *sumsq;       // RmsNorm: each split's sums of squares of x [split][m], or NULL
     const float *a0;
     void *out;
-    uint32_t splits, m, n, stages;
+    uint32_t splits, m, n, k, stages;
+    float eps;
     int out_bf16, pair_sum;
     ts_after after;
 };

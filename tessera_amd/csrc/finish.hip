@@ -32,8 +32,14 @@ __global__ __launch_bounds__(256) void split_finish_kernel(SplitSum p) {
                 if (PAIR) u += tu[j];
             }
     }
-    const float head = p.head ? *p.head : 1.0f;
-    const uint32_t n = (uint32_t)(i % p.n);
+    float head = p.head ? *p.head : 1.0f;
+    const uint32_t n = (uint32_t)(i % p.n);  // V divides n: one row
+    if (p.sumsq) {
+        const uint32_t m = (uint32_t)(i / p.n);
+        float ss = 0.0f;
+        for (uint32_t s = 0; s < p.splits; s++) ss += p.sumsq[s * p.m + m];
+        head = 1.0f / sqrtf(ss / (float)p.k + p.eps);
+    }
 #pragma unroll
     for (int e = 0; e < V; e++) {
         float a = g[e] * head, b = u[e] * head;

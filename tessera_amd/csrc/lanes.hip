@@ -1,5 +1,6 @@
 // "lanes": out[m, n] = after(sum_k x[m, k] w[n, k]) for m <= 64 rows.
-// Rows 1..4 go to the vector-ALU kernel in gemv.hip; 5..64 run here.
+// Rows 1..4 go to the vector-ALU kernel in gemv.hip; of 5..64 rows, products of whole units
+// go to stream.hip and the rest (any k, small weights) run here.
 //
 // Replaces the reference's few-row matmul rules: lanes (a 32-lane group per
 // column, engine/rules/linear/src/lanes.rs:17-143) and thin (a thread per
@@ -434,18 +435,23 @@ int check(const ts_linear_args *a) {
 extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
     if (a && (a->stages & TS_AFTER_ARGMAX)) return (size_t)a->m * 8;  // the keys
     if (!a || a->m <= 4 || a->m > 64) return 0;
-    if (ts::block_form(a->w_dtype)) return ts::block_lanes_workspace(a);
+    if (ts::block_form(a->w_dtype)) return ts::stream_fits(a) ? ts::stream_workspace(a) : 0;
     const Plan pl = plan(a);
-    if (pl.splits <= 1) return 0;
     const size_t per = (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1);
-    return (size_t)pl.splits * per * sizeof(float);
+    const size_t here = pl.splits <= 1 ? 0 : (size_t)pl.splits * per * sizeof(float);
+    // Never less than this file's kernel takes: fewer rows of the same product may run here,
+    // and its need grows with the rows, so the size for the most rows serves them all.
+    return ts::stream_fits(a) ? std::max(here, ts::stream_workspace(a)) : here;
 }
 
 extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
     if (a && ts::block_form(a->w_dtype)) {
         if (a->m <= 4) return ts::block_gemv_launch(a, stream);
-        const int few = ts::block_lanes_launch(a, stream);
-        return few != 1 ? few : ts::block_tiled_launch(a, stream);
+        const int bad = ts::block_check(a, "tiled");
+        if (bad) return bad;
+        if ((a->stages & ~(TS_AFTER_ADD | TS_AFTER_SILU_MUL)) || !ts::stream_fits(a))
+            return ts::block_tiled_launch(a, stream);
+        return ts::stream_launch(a, stream);
     }
     int rc = check(a);
     if (rc) return rc;
@@ -454,6 +460,7 @@ extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
         rc = ts::linear_after(a, "lanes", &c);
         return rc ? rc : ts::gemv_launch(a, stream);
     }
+    if (ts::stream_fits(a)) return ts::stream_launch(a, stream);
     const Plan pl = plan(a);
     const size_t need = tessera_hip_lanes_workspace(a);
     if (need && (!a->workspace || a->workspace_bytes < need))

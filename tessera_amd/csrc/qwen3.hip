@@ -293,10 +293,9 @@ size_t workspace_need(ts_qwen3 *m) {
     const uint32_t H = c.hidden, D = c.head_dim;
     const uint32_t shapes[][2] = {{(c.heads + 2 * c.kv_heads) * D, H}, {H, c.heads * D}, {c.ffn, H},
                                   {H, c.ffn}, {c.vocab, H}};
-    // Split partials grow with the rows: size for one row and for the most rows a
-    // launch can carry to the few-row kernels (up to 64).
-    const uint32_t row_counts[] = {1, std::min<uint32_t>(c.max_prompt, 64)};
-    for (uint32_t rows : row_counts)
+    // The most split sums of any row count that a launch can carry to the few-row kernels
+    // (up to 64; fewer rows may be split more ways).
+    for (uint32_t rows = 1; rows <= std::min<uint32_t>(c.max_prompt, 64); rows++)
         for (auto &sh : shapes) {
             ts_linear_args a = lin(nullptr, nullptr, nullptr, rows, sh[0], sh[1], m);
             if (sh[0] == c.ffn && sh[1] == H) a.stages = TS_AFTER_SILU_MUL;

@@ -1,0 +1,78 @@
+"""bf16 and e4m3 weights streamed at 5..64 rows (whole units of k): the edges of the row
+tiles, of the 32 weight rows a wave, of a last step that holds fewer units than slices, and
+split k, with every operand form and epilogue, within product_bound of the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+from tests.helpers import from_dev, linear_bound, rng, to_dev
+from tests.test_gpu_pipe import operands
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+FORMS = [("f32", "bf16"), ("bf16", "bf16"), ("f32", "e4m3"), ("bf16", "e4m3")]
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("m,n,k", [(5, 33, 128), (16, 130, 384), (17, 31, 640), (33, 200, 1152), (48, 1000, 256),
+                                   (64, 65, 4096), (9, 2500, 1024)])
+def test_stream_edges(m, n, k, x, w):
+    from tessera_amd import rules as R
+    print(f"stream {x} {w} m={m} n={n} k={k}", flush=True)
+    r = rng(m + n + k)
+    xd, wd, sd, xf, wf, want = operands(r, m, n, k, x, w)
+    bound = linear_bound(xf, wf)
+    res = r.standard_normal((m, n)).astype(np.float32)
+    got = from_dev(R.linear(xd, wd, w_scale=sd, a0=to_dev(res, torch)))
+    assert np.all(np.abs(got.astype(np.float64) - (want + res)) <= bound + 1e-6)
+    got32 = from_dev(R.linear(xd, wd, w_scale=sd))
+    got16 = from_dev(R.linear(xd, wd, w_scale=sd, out_dtype=torch.bfloat16))
+    assert np.array_equal(got16, O.bf16_widen(O.bf16_narrow(got32)))
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("m,n,k", [(6, 50, 192), (20, 70, 1024), (64, 130, 2176)])
+def test_stream_gate_up(m, n, k, x, w):
+    from tessera_amd import rules as R
+    if w == "e4m3":
+        k = k // 128 * 128
+    r = rng(m + n)
+    xd, wd, sd, xf, wf, gu = operands(r, m, 2 * n, k, x, w)
+    g, u = gu[:, :n], gu[:, n:]
+    want = O.act("silu", g) * u
+    b = linear_bound(xf, wf)
+    got = from_dev(R.linear(xd, wd, w_scale=sd, silu_mul=True))
+    assert np.all(np.abs(got.astype(np.float64) - want) <= 1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5)
+
+
+@pytest.mark.parametrize("w", ["bf16", "e4m3"])
+@pytest.mark.parametrize("m,n,k", [(5, 40, 128), (7, 33, 384), (16, 100, 4096), (11, 20000, 1024)])
+def test_stream_norm(m, n, k, w):
+    """RmsNorm before the product, one group and several along k and the columns (the first
+    two have a last step of fewer units)."""
+    from tessera_amd import rules as R
+    r = rng(m * n)
+    xd, wd, sd, xf, wf, _ = operands(r, m, n, k, "f32", w)
+    g = (1 + 0.1 * r.standard_normal(k)).astype(np.float32)
+    xn = O.rms_norm(xf * 3, g, 1e-6)
+    want = xn.astype(np.float64) @ wf.T.astype(np.float64)
+    got = from_dev(R.linear(xd * 3, wd, w_scale=sd, gain=to_dev(g, torch), eps=1e-6))
+    assert np.all(np.abs(got - want) <= 2 * linear_bound(xn, wf))
+
+
+def test_stream_without_workspace():
+    """No workspace: the same product with k unsplit, the norm's sums included."""
+    from tessera_amd import abi, rules as R
+    r = rng(8)
+    m, n, k = 12, 256, 4096
+    xd, wd, _, xf, wf, _ = operands(r, m, n, k, "f32", "bf16")
+    g = np.ones(k, np.float32)
+    gd, out = to_dev(g, torch), torch.empty((m, n), device="cuda")
+    a = R.linear_args(xd, wd, out, gain=gd, stages=abi.TS_BEFORE_RMS_NORM)
+    assert abi.load().tessera_hip_linear_workspace(C.byref(a)) > 0  # k is split where it may be
+    abi.call("tessera_hip_linear", C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    xn = O.rms_norm(xf, g, 1e-6)
+    assert np.all(np.abs(from_dev(out) - xn.astype(np.float64) @ wf.T) <= 2 * linear_bound(xn, wf))
