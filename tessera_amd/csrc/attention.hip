@@ -437,15 +437,16 @@ __global__ __launch_bounds__(kLongWaves * 64) void attend_long_kernel(RowsParams
     const uint32_t w0 = g0 + wave * 32 * iters;  // this wave's first key
 
     // Block at kb (clamped into [0, pos] so its page exists): K 4 x 16B per lane (key
-    // col, d 32 grp..+32), V 4 x 16B (key 4j + grp, d 8 col..+8).
+    // col, d 32 j + 8 grp..+8: the four lanes of a key read 64 contiguous bytes a load), V 4
+    // x 16B (key 4j + grp, d 8 col..+8).
     auto load = [&](uint32_t kb, u32x4 (&kk)[4], u32x4 (&vq)[4]) {
         const uint32_t kbc = min(kb, pos) & ~15u;
         const uint64_t row0 = p.table ? (((uint64_t)stab[(kbc >> p.page_shift) - p0] << p.page_shift) | (kbc & pmask))
                                       : (uint64_t)slot * p.keys + kbc;
         const uint32_t room = p.table ? 15u : p.keys - 1 - min(kbc, p.keys - 1);
-        const uint16_t *kr = p.k + ((row0 + min(col, room)) * p.kv_heads + kvh) * 128 + 32 * grp;
+        const uint16_t *kr = p.k + ((row0 + min(col, room)) * p.kv_heads + kvh) * 128 + 8 * grp;
 #pragma unroll
-        for (int j = 0; j < 4; j++) kk[j] = *((const u32x4 *)kr + j);
+        for (int j = 0; j < 4; j++) kk[j] = *((const u32x4 *)kr + 4 * j);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const uint32_t i = 4 * j + grp;
@@ -460,10 +461,10 @@ __global__ __launch_bounds__(kLongWaves * 64) void attend_long_kernel(RowsParams
     u32x4 qh[4], ql[4];
     {
         const bool ok = col < G;
-        const float4 *qr = (const float4 *)(p.q + ((size_t)r * p.heads + kvh * G + (ok ? col : 0)) * 128 + 32 * grp);
+        const float4 *qr = (const float4 *)(p.q + ((size_t)r * p.heads + kvh * G + (ok ? col : 0)) * 128 + 8 * grp);
         float4 qv[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) qv[i] = qr[i];
+        for (int i = 0; i < 8; i++) qv[i] = qr[8 * (i >> 1) + (i & 1)];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float f[8] = {qv[2 * j].x, qv[2 * j].y, qv[2 * j].z, qv[2 * j].w,

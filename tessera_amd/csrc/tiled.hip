@@ -33,9 +33,6 @@
 
 namespace {
 
-#ifndef TS_PIPE_SMALL
-#define TS_PIPE_SMALL 256
-#endif
 constexpr int BM = 128, BN = 128, BK = 64;  // the default tile; BT = 64 for products with few tiles
 constexpr int kThreads = 256;
 
@@ -368,7 +365,7 @@ struct Pipe {
     static constexpr int NA = TM / A::RPI / 4;  // A load instructions per wave per stage
     static constexpr int NB = TN / B::RPI / 4;  // B load instructions per wave per stage
     static constexpr int A_BYTES = TM * A::CPR * 16, STAGE = A_BYTES + TN * B::CPR * 16, LDS = NS * STAGE;
-    static constexpr int GM = XF32 ? 4 : 2, GN = 4 / GM;  // waves along the rows and the columns
+    static constexpr int GM = TM == 32 ? 1 : XF32 ? 4 : 2, GN = 4 / GM;  // waves along the rows and the columns
     static constexpr int WM = TM / GM, WN = TN / GN, FI = WM / 16, FJ = WN / 16;
     static_assert(NA >= 1 && NB >= 1 && FI >= 1 && (KD == 64 || (KD == 32 && !W8)), "pipe shape");
 };
@@ -792,6 +789,14 @@ int pipe_wide(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
     return pipe_launch<128, 128, 64, 3, false, true, PICK>(p, silu, stream);
 }
 
+// 32 x 128 tiles for matrices of few rows: the four waves side by side along the columns.
+int pipe_few(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
+    if (xf) return w8 ? pipe_launch<32, 128, 64, 3, true, true, true>(p, silu, stream)
+                      : pipe_launch<32, 128, 64, 3, true, false, true>(p, silu, stream);
+    return w8 ? pipe_launch<32, 128, 64, 4, false, true, true>(p, silu, stream)
+              : pipe_launch<32, 128, 64, 4, false, false, true>(p, silu, stream);
+}
+
 using Kern = void (*)(TiledParams);
 
 template <int BT, bool XF32, bool W8, bool PICK>
@@ -863,7 +868,7 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
         const bool wide = ((tiles192 + 511) / 512) * 3 < ((tiles + 511) / 512) * 2;
         // A stage chain takes 64 x 64 tiles: at 128 x 128 its values and sums spill.
         if (p.after.count) return pipe_small<true>(p, xf, w8, silu, stream);
-        if (tiles < TS_PIPE_SMALL) return pipe_small<false>(p, xf, w8, silu, stream);
+        if (tiles < 256) return pipe_small<false>(p, xf, w8, silu, stream);
         if (xf || w8) return pipe_wide<false>(p, xf, w8, silu, stream);
         if (wide) return pipe_launch<128, 192, 64, 2, false, false, false>(p, silu, stream);
         return pipe_launch<128, 128, 64, 2, false, false, false>(p, silu, stream);
@@ -909,8 +914,15 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     if (!a->workspace || a->workspace_bytes < need)
         return ts::fail(TS_ERR_WORKSPACE, "picked: workspace %zu bytes, need %zu", a->workspace_bytes, need);
     TS_REQUIRE(ts::aligned(a->workspace, 4), "picked: workspace must be 4-byte aligned");
+    const bool xf = a->x_dtype == TS_F32, w8 = a->w_dtype == TS_E4M3;
+    const bool pipe = pipe_fits((a->rows - 1) / a->repeat + 1, a->k, xf ? 4 : 2) && !(a->after && a->after->count);
+    // Up to 16 rows a matrix on average 32-row tiles: most matrices have one tile either way,
+    // and a 128-row one loads its few rows 128 / rows times over beside the weights. 128
+    // matrices of 4096 x 1536 at 1 / 16 rows each 213 -> 186 / 324 -> 319 us (2 x 1536 x 4096
+    // 374 -> 373 / 575 -> 570: HBM), at 32 rows 350 -> 369; one token's 8 matrices 62 -> 41.
+    const bool few = pipe && a->rows <= 16ull * a->count;
     ts::Route route;
-    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, BM, a->workspace, &route, stream);
+    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, few ? 32 : BM, a->workspace, &route, stream);
     if (rc) return rc;
     const bool silu = a->stages & TS_AFTER_SILU_MUL;
     TiledParams p;
@@ -929,8 +941,8 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // A stage chain takes the register-staged kernel (the pipelined one's chain variant spills).
     // 128 x 192 tiles where the columns divide evenly (fewer re-reads of the gathered
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
-    const bool xf = a->x_dtype == TS_F32, w8 = a->w_dtype == TS_E4M3;
-    if (pipe_fits((a->rows - 1) / a->repeat + 1, a->k, xf ? 4 : 2) && !p.after.count) {
+    if (few) return pipe_few(p, xf, w8, silu, stream);
+    if (pipe) {
         if (xf || w8) return pipe_wide<true>(p, xf, w8, silu, stream);
         if ((silu ? a->n % 96 : a->n % 192) == 0)
             return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);

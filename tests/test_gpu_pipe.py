@@ -68,17 +68,21 @@ def test_pipe_gate_up(m, n, k, x, w):
     assert np.all(np.abs(got.astype(np.float64) - want) <= 1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5)
 
 
-@pytest.mark.parametrize("x,w", FORMS)
-@pytest.mark.parametrize("silu", [False, True])
-def test_pipe_picked(x, w, silu):
-    """Expert products on the same tiles: matrices of 0, 1, 128, 129 and more rows, ids
-    outside the set."""
+@pytest.mark.parametrize("x,w", FORMS + [("bf16", "bf16")])
+@pytest.mark.parametrize("silu,counts", [
+    (False, ((0, 1), (1, 128), (2, 129), (4, 300), (5, 17), (9, 6))),
+    (True, ((0, 1), (1, 128), (2, 129), (4, 300), (5, 17), (9, 6))),
+    (False, ((0, 1), (1, 31), (3, 32), (4, 20), (9, 2))),
+    (True, ((0, 33), (2, 16), (5, 17), (8, 1)))])
+def test_pipe_picked(x, w, silu, counts):
+    """Expert products on the same tiles: matrices of 0, 1, 128, 129 and more rows, and on 32-row
+    tiles (16 rows a matrix on average) of 0 to 33; ids outside the set."""
     from tessera_amd import rules as R
     r = rng(17 + silu)
     count, n, k, offset = 6, 72, 128, 3
     used = 2 * n if silu else n
     stride = used + 5
-    ids = np.concatenate([np.full(c, e) for e, c in ((0, 1), (1, 128), (2, 129), (4, 300), (5, 17), (9, 6))])
+    ids = np.concatenate([np.full(c, e) for e, c in counts])
     ids = r.permutation(ids).astype(np.uint32)
     rows = len(ids)
     xd, wd, sd, xf, wf, _ = operands(r, rows, count * stride, k, x, w)
