@@ -229,4 +229,12 @@ def check(code: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    code = getattr(_lib or load(), name)(*args)
+    if code != TS_OK:
+        check(code, name)
+
+
+def workspace_of(name: str, args) -> int:
+    """The bytes the entry point's *_workspace() reports, 0 where it has none."""
+    fn = getattr(load(), name + "_workspace", None)
+    return fn(C.byref(args)) if fn is not None and name + "_workspace" in SIGNATURES else 0

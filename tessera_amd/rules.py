@@ -22,11 +22,12 @@ _DT = {torch.float32: abi.TS_F32, torch.bfloat16: abi.TS_BF16, torch.uint8: abi.
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # The handle of torch.cuda.current_stream(), without the Stream object around it.
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 class Workspace:
@@ -90,17 +91,13 @@ def chain(stages, operands=(), *, sum_at=0, spans=None):
 
 def linear_args(x, w, out, *, w_scale=None, gain=None, a0=None, stages=0, eps=1e-6, w_form=None):
     m, k = x.shape
-    n = out.shape[1]
-    a = abi.LinearArgs()
-    a.x, a.w, a.w_scale, a.gain, a.a0, a.out = (_ptr(x), _ptr(w), _ptr(w_scale), _ptr(gain), _ptr(a0),
-                                                _ptr(out))
-    a.m, a.n, a.k = m, n, k
-    a.x_dtype, a.out_dtype = _DT[x.dtype], _DT[out.dtype]
     # Block forms: w is the packed tensor (uint8: head, then each row's blocks).
-    a.w_dtype = (abi.TS_F32_PARTS if w_form == "f32_parts" else BLOCK_FORMS[w_form]) if w_form is not None \
-        else _DT[w.dtype]
-    a.stages, a.eps = stages, eps
-    return a
+    w_dtype = _DT[w.dtype] if w_form is None else abi.TS_F32_PARTS if w_form == "f32_parts" else BLOCK_FORMS[w_form]
+    # One call with every field in order: a ctypes attribute at a time costs more than the launch.
+    return abi.LinearArgs(x.data_ptr(), w.data_ptr(), None if w_scale is None else w_scale.data_ptr(),
+                          None if gain is None else gain.data_ptr(), None if a0 is None else a0.data_ptr(),
+                          out.data_ptr(), None, 0, m, out.shape[1], k, _DT[x.dtype], w_dtype, _DT[out.dtype], stages,
+                          eps)
 
 
 def _linear(fn: str, x, w, *, out=None, out_dtype=torch.float32, w_scale=None, gain=None, a0=None,
@@ -119,12 +116,13 @@ def _linear(fn: str, x, w, *, out=None, out_dtype=torch.float32, w_scale=None, g
     a = linear_args(x, w, out, w_scale=w_scale, gain=gain, a0=a0, stages=stages, eps=eps, w_form=w_form)
     if after is not None:
         a.after = C.addressof(after)
-    lib = abi.load()
-    need = getattr(lib, fn + "_workspace")(C.byref(a)) if hasattr(lib, fn + "_workspace") else 0
-    # The split sums' scratch is the call's own (the allocator's cache keeps it in stream
-    # order), so products on several streams or threads do not share it.
-    scratch = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-    a.workspace, a.workspace_bytes = _ptr(scratch), need
+    if m > 4:  # the products of fewer rows take no workspace
+        need = abi.workspace_of(fn, a)
+        if need:
+            # The split sums' scratch is the call's own (the allocator's cache keeps it in stream
+            # order), so products on several streams or threads do not share it.
+            scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+            a.workspace, a.workspace_bytes = scratch.data_ptr(), need
     abi.call(fn, C.byref(a), _stream())
     return out
 
