@@ -134,7 +134,9 @@ typedef struct {
 } ts_linear_args;
 
 /* Picks `lanes` for m <= 64 and `tiled` otherwise (the cost select of
- * engine/plan/lower/src/cost.rs between the two rules). */
+ * engine/plan/lower/src/cost.rs between the two rules). Where the tiles alone leave CUs
+ * idle, k is split across groups with the workspace that the query names; without it the
+ * product runs unsplit. */
 int tessera_hip_linear(const ts_linear_args *a, void *stream);
 size_t tessera_hip_linear_workspace(const ts_linear_args *a);
 

@@ -157,7 +157,9 @@ ts_linear_args lin(const void *x, const void *w, void *out, uint32_t rows, uint3
     memset(&a, 0, sizeof a);
     a.x = x; a.w = w; a.out = out; a.m = rows; a.n = n; a.k = k;
     a.x_dtype = TS_F32; a.w_dtype = TS_BF16; a.out_dtype = TS_F32;
-    a.workspace = m->ws; a.workspace_bytes = m->ws_bytes;
+    // Longer prompts run unsplit: the sums of a row then do not depend on how many rows the
+    // prompt has (a split of the o and down products is worth 2% of a 1000-token prefill).
+    a.workspace = rows <= 64 ? m->ws : nullptr; a.workspace_bytes = rows <= 64 ? m->ws_bytes : 0;
     a.eps = m->c.eps;
     return a;
 }

@@ -53,6 +53,8 @@ struct TiledParams {
     uint32_t matrices, repeat, stride, offset;
     ts_after after;  // stage chain (count 0: none)
     int pair_sum;    // TS_F32_PARTS: the second row block is the low parts; the output sums the pair
+    uint32_t splits;     // pipelined tiles: groups along k; more than 1: raw sums to part
+    float *part;         // [split][gate, up or one][m][n]
     uint32_t pick_cols;  // PICK on the pipelined tiles: column tiles (0: a 2-D grid of them)
 };
 
@@ -405,7 +407,11 @@ TS_DEV void pipe_wait_ahead(uint32_t ahead) {
     }
 }
 
-template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, bool CHAIN>
+// What a pipelined kernel does with its sums: its epilogue, the epilogue with a stage chain (64
+// x 64 tiles only: larger ones would spill), or raw sums of a split of k to memory.
+enum Ends { kPlain, kChain, kSplit };
+
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tiled_pipe_kernel(TiledParams p) {
     using P = Pipe<TM, TN, KD, NS, XF32, W8>;
     extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: two groups share a CU
@@ -413,15 +419,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint32_t wm = wave / P::GN, wn = wave % P::GN;
     const uint32_t col = lane & 15, grp = lane >> 4;
     constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
-    uint32_t tx = blockIdx.x, ty = blockIdx.y;
+    uint32_t tx = blockIdx.x, ty = blockIdx.y, split = 0;
     if (!PICK) {
         // XCD-aware order (one-dimensional grid): group b runs on XCD b % 8, and XCD x
         // takes the x-th eighth of the tiles, walked in bands of kBand tile rows column
         // by column, so the groups an XCD runs at once share rows and weight columns
         // in its L2.
-        const uint32_t gx = p.stride, gy = p.offset, tiles = gx * gy, per = (tiles + 7) / 8;
-        const uint32_t t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-        if (t >= tiles) return;
+        // A split of k is a grid of tiles of its own, behind the one before it.
+        const uint32_t gx = p.stride, gy = p.offset, tiles = gx * gy, all = END == kSplit ? tiles * p.splits : tiles,
+                       per = (all + 7) / 8;
+        uint32_t t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+        if (t >= all) return;
+        if (END == kSplit) {
+            split = t / tiles;
+            t -= split * tiles;
+        }
         const uint32_t band = t / (kBand * gx), rows = min(kBand, gy - band * kBand);
         const uint32_t within = t - band * kBand * gx;
         ty = band * kBand + within % rows;
@@ -535,13 +547,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int j = 0; j < P::FJ; j++) acc[i][j] = f32x4{0, 0, 0, 0};
 
-    const uint32_t steps = p.k / KD;
+    uint32_t s0 = 0, steps = p.k / KD;
+    if (END == kSplit) {
+        const uint32_t each = steps / p.splits, more = steps - each * p.splits;  // the first `more` take one more
+        s0 = split * each + min(split, more);
+        steps = each + (split < more ? 1 : 0);
+    }
     // 16-row fragments of this wave that hold a row of the tile (wave-uniform).
     const uint32_t wrow0 = m0 + wm * P::WM;
     const uint32_t live_frags = mend > wrow0 ? min((mend - wrow0 + 15) / 16, (uint32_t)P::FI) : 0u;
 #pragma unroll
     for (int s = 0; s < NS - 1; s++)
-        if ((uint32_t)s < steps) fetch(s, s * KD);
+        if ((uint32_t)s < steps) fetch(s, (s0 + s) * KD);
     // The matrix work of the stage in slot `at`.
     auto multiply = [&](uint32_t at) {
         const char *sa = lds + at * P::STAGE, *sb = sa + P::A_BYTES;
@@ -599,7 +616,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     uint32_t s = 0, at = 0, fill = NS - 1;  // the slots of this step and of the stage loaded in it
     for (; s + NS - 1 < steps; s++) {
         pipe_wait<(P::NA + P::NB) * (NS - 2)>();
-        fetch(fill, (s + NS - 1) * KD);
+        fetch(fill, (s0 + s + NS - 1) * KD);
         multiply(at);
         at = at == NS - 1 ? 0 : at + 1;
         fill = fill == NS - 1 ? 0 : fill + 1;
@@ -616,6 +633,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint32_t N = p.n;
     constexpr int JO = SILU ? P::FJ / 2 : P::FJ;
     constexpr uint32_t WO = SILU ? P::WN / 2 : P::WN;
+    if (END == kSplit) {  // raw sums; split_finish adds the splits and runs the epilogue
+        const size_t mn = (size_t)p.m * N;
+        float *dst = p.part + (size_t)split * (SILU ? 2 : 1) * mn;
+#pragma unroll
+        for (int i = 0; i < P::FI; i++) {
+            const uint32_t m = m0 + wm * P::WM + i * 16 + col;
+            if (m >= p.m) continue;
+#pragma unroll
+            for (int j = 0; j < P::FJ; j++) {
+                const uint32_t n = n0 + wn * WO + j % JO * 16 + 4 * grp;
+                float *o = dst + (j < JO ? 0 : mn) + (size_t)m * N + n;
+                if ((N & 3) == 0 && n < N) __builtin_nontemporal_store(acc[i][j], (f32x4 *)o);
+                else
+                    for (uint32_t r = 0; r < 4 && n + r < N; r++) o[r] = acc[i][j][r];
+            }
+        }
+        return;
+    }
     // e4m3: each weight row's scale on its finished sums.
     if (W8) {
 #pragma unroll
@@ -682,7 +717,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < JO; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++) val[i][j][r] = value(i, j, r);
-    if (CHAIN) {  // the chain's variant: its values and sums need more registers
+    if (END == kChain) {  // the chain's variant: its values and sums need more registers
         // Value e = (i JO + j) 4 + r: row fragment i, column fragment j, column 4 grp + r.
         auto row_of = [&](int e) {
             const uint32_t tr = wm * P::WM + (e / (4 * JO)) * 16 + col;
@@ -725,17 +760,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 }
 
-// CHAIN: the instance that runs stage chains (64 x 64 tiles only: larger ones would spill).
-template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool PICK, bool CHAIN = false>
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool PICK, Ends END = kPlain>
 int pipe_launch(TiledParams p, bool silu, void *stream) {
     constexpr int lds = Pipe<TM, TN, KD, NS, XF32, W8>::LDS;
-    const void *k = silu ? (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, CHAIN>
-                         : (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, CHAIN>;
+    const void *k = silu ? (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END>
+                         : (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END>;
     // The dynamic LDS size is raised once per kernel (thread-safe static initialisation).
     static const hipError_t attr[2] = {
-        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, CHAIN>,
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, CHAIN>,
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
     if (attr[silu]) return ts::hip_status(attr[silu], "tiled (pipelined): LDS attribute");
     const uint32_t oc = silu ? TN / 2 : TN;
@@ -758,7 +792,7 @@ int pipe_launch(TiledParams p, bool silu, void *stream) {
         const uint32_t gy = (p.m + TM - 1) / TM;
         p.stride = gx;
         p.offset = gy;
-        grid = dim3(8 * (uint32_t)(((uint64_t)gx * gy + 7) / 8));
+        grid = dim3(8 * (uint32_t)(((uint64_t)gx * gy * p.splits + 7) / 8));
     }
     void *args[] = {(void *)&p};
     const hipError_t e = hipLaunchKernel(k, grid, dim3(kThreads), args, lds, (hipStream_t)stream);
@@ -773,20 +807,21 @@ bool pipe_fits(uint32_t x_rows, uint32_t k, uint32_t x_bytes) {
 }
 
 // 64 x 64 tiles, four stages of 16 KiB or three of 20 to 24.
-template <bool CHAIN>
+template <Ends END>
 int pipe_small(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
-    if (xf) return w8 ? pipe_launch<64, 64, 64, 3, true, true, false, CHAIN>(p, silu, stream)
-                      : pipe_launch<64, 64, 64, 3, true, false, false, CHAIN>(p, silu, stream);
-    return w8 ? pipe_launch<64, 64, 64, 4, false, true, false, CHAIN>(p, silu, stream)
-              : pipe_launch<64, 64, 64, 4, false, false, false, CHAIN>(p, silu, stream);
+    if (xf) return w8 ? pipe_launch<64, 64, 64, 3, true, true, false, END>(p, silu, stream)
+                      : pipe_launch<64, 64, 64, 3, true, false, false, END>(p, silu, stream);
+    return w8 ? pipe_launch<64, 64, 64, 4, false, true, false, END>(p, silu, stream)
+              : pipe_launch<64, 64, 64, 4, false, false, false, END>(p, silu, stream);
 }
 
-// 128 x 128 tiles of f32 rows or e4m3 weights.
-template <bool PICK>
+// 128 x 128 tiles.
+template <bool PICK, Ends END = kPlain>
 int pipe_wide(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
-    if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK>(p, silu, stream)
-                      : pipe_launch<128, 128, 32, 3, true, false, PICK>(p, silu, stream);
-    return pipe_launch<128, 128, 64, 3, false, true, PICK>(p, silu, stream);
+    if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK, END>(p, silu, stream)
+                      : pipe_launch<128, 128, 32, 3, true, false, PICK, END>(p, silu, stream);
+    return w8 ? pipe_launch<128, 128, 64, 3, false, true, PICK, END>(p, silu, stream)
+              : pipe_launch<128, 128, 64, 2, false, false, PICK, END>(p, silu, stream);
 }
 
 // 32 x 128 tiles for matrices of few rows: the four waves side by side along the columns.
@@ -813,7 +848,41 @@ Kern pick_kernel(bool xf, bool w8, bool silu, bool chain) {
 
 }  // namespace
 
-extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
+namespace {
+
+// The k split of a product of more than 64 rows whose tiles alone leave CUs idle: times in
+// us, from what the pipelined tiles take a 64-deep step (64 x 64 0.4, f32 rows 0.5 with one
+// group a CU and 0.7 with two; 128 x 128 0.9 and 1.7) and what the second kernel takes (4 us and
+// its sums' way to memory and back at 5 TB/s); a split has to promise 15%. Measured: 128 f32 rows by 1024 x 3072 23.8 -> 11.6
+// us, 300 bf16 rows by e4m3 4096 x 14336 69 -> 52, 500 by bf16 2560 x 9728 59 -> 40, 1200 f32 rows
+// by 2048 x 8192 129 -> 91; 1000 f32 rows by 1024 x 3072 24.8 against 26.8 split in two.
+struct Split {
+    uint32_t splits;
+    bool wide;  // 128 x 128 tiles
+};
+
+Split plan_split(const ts_linear_args *a) {
+    const bool pair = (a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS, xf = a->x_dtype == TS_F32;
+    const uint32_t steps = a->k / 64;
+    Split best = {1, false};
+    auto tiles = [&](uint32_t t) { return (uint64_t)((a->n + (pair ? t / 2 : t) - 1) / (pair ? t / 2 : t)) * ((a->m + t - 1) / t); };
+    const float sums = 8e-6f / 5 * (float)a->m * (float)a->n * (pair ? 2 : 1);
+    auto cost = [&](bool wide, uint32_t s) {
+        const uint64_t rounds = (tiles(wide ? 128 : 64) * s + 511) / 512;
+        return (float)rounds * ((steps + s - 1) / s + 1) * (wide ? (xf ? 1.7f : 0.9f) : !xf ? 0.4f : tiles(64) * s > 256 ? 0.7f : 0.5f) + (s > 1 ? 4.0f + (s + 1) * sums : 0.0f);
+    };
+    if (tiles(64) > 1024) return best;  // enough tiles of some size
+    float least = 0.85f * cost(tiles(128) >= 256, 1);
+    for (int wide = 0; wide < 2; wide++)
+        for (uint32_t s = 2; s <= 16 && 4 * s <= steps; s++)
+            if (cost(wide, s) < least) {
+                least = cost(wide, s);
+                best = {s, wide != 0};
+            }
+    return best;
+}
+
+int tiled(const ts_linear_args *a, bool may_split, void *stream) {
     if (a && ts::block_form(a->w_dtype)) return ts::block_tiled_launch(a, stream);
     TS_REQUIRE(a && a->x && a->w && a->out, "tiled: null pointer");
     TS_REQUIRE(a->m >= 1 && a->n >= 1 && a->k >= 1, "tiled: empty product m=%u n=%u k=%u", a->m, a->n, a->k);
@@ -854,7 +923,24 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
     p.perm = p.row_start = p.tile_start = nullptr;
     p.matrices = 0; p.repeat = 1; p.stride = 0; p.offset = 0;
     const bool xf = a->x_dtype == TS_F32, w8 = w_dtype == TS_E4M3;
+    p.splits = 1;
+    p.part = nullptr;
     if (pipe_fits(0, a->k, 4)) {
+        const Split sp = may_split ? plan_split(a) : Split{1, false};
+        const size_t need = sp.splits <= 1 ? 0 : (size_t)sp.splits * a->m * a->n * (silu ? 2 : 1) * sizeof(float);
+        if (need && a->workspace && a->workspace_bytes >= need && ts::aligned(a->workspace, 16)) {
+            p.splits = sp.splits;
+            p.part = (float *)a->workspace;
+            const ts_after after = p.after;
+            p.after.count = 0;  // the second kernel's
+            rc = sp.wide ? pipe_wide<false, kSplit>(p, xf, w8, silu, stream) : pipe_small<kSplit>(p, xf, w8, silu, stream);
+            if (rc) return rc;
+            ts::SplitSum f = {};
+            f.part = p.part; f.splits = p.splits; f.out = a->out; f.a0 = a->a0;
+            f.w_scale = w8 ? p.w_scale : nullptr; f.pair_sum = parts;
+            f.m = a->m; f.n = a->n; f.k = a->k; f.stages = a->stages; f.out_bf16 = p.out_bf16; f.after = after;
+            return ts::split_finish(f, stream);
+        }
         // 128 x 128 tiles from one tile per CU up (fewer, larger tiles read less per
         // flop), 64 x 64 below that (measured on the 2048-row projections: q with 256
         // tiles of 128 runs 1.15x faster than with 1024 of 64; o, kv and down with 128
@@ -867,11 +953,10 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
         const uint64_t tiles192 = (a->n + oc * 3 / 2 - 1) / (oc * 3 / 2) * ((a->m + 127) / 128);
         const bool wide = ((tiles192 + 511) / 512) * 3 < ((tiles + 511) / 512) * 2;
         // A stage chain takes 64 x 64 tiles: at 128 x 128 its values and sums spill.
-        if (p.after.count) return pipe_small<true>(p, xf, w8, silu, stream);
-        if (tiles < 256) return pipe_small<false>(p, xf, w8, silu, stream);
-        if (xf || w8) return pipe_wide<false>(p, xf, w8, silu, stream);
-        if (wide) return pipe_launch<128, 192, 64, 2, false, false, false>(p, silu, stream);
-        return pipe_launch<128, 128, 64, 2, false, false, false>(p, silu, stream);
+        if (p.after.count) return pipe_small<kChain>(p, xf, w8, silu, stream);
+        if (tiles < 256) return pipe_small<kPlain>(p, xf, w8, silu, stream);
+        if (wide && !xf && !w8) return pipe_launch<128, 192, 64, 2, false, false, false>(p, silu, stream);
+        return pipe_wide<false>(p, xf, w8, silu, stream);
     }
     const bool chain = p.after.count;
     Kern k = bt == 64 ? pick_kernel<64, false>(xf, w8, silu, chain) : pick_kernel<128, false>(xf, w8, silu, chain);
@@ -879,6 +964,10 @@ extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) {
     TS_CHECK_LAUNCH("tiled launch");
     return TS_OK;
 }
+
+}  // namespace
+
+extern "C" int tessera_hip_tiled(const ts_linear_args *a, void *stream) { return tiled(a, false, stream); }
 
 static int picked_check(const ts_picked_args *a) {
     TS_REQUIRE(a && a->x && a->w && a->ids && a->out, "picked: null pointer");
@@ -927,6 +1016,8 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     const bool silu = a->stages & TS_AFTER_SILU_MUL;
     TiledParams p;
     p.pick_cols = 0;
+    p.splits = 1;
+    p.part = nullptr;
     p.pair_sum = 0;
     ts::after_check(a->after, true, "picked", &p.after);
     rc = ts::zero_absent_launch(route, a->count, a->out, a->n, a->out_dtype == TS_BF16, p.after, stream);
@@ -943,10 +1034,9 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
     if (few) return pipe_few(p, xf, w8, silu, stream);
     if (pipe) {
-        if (xf || w8) return pipe_wide<true>(p, xf, w8, silu, stream);
-        if ((silu ? a->n % 96 : a->n % 192) == 0)
+        if (!xf && !w8 && (silu ? a->n % 96 : a->n % 192) == 0)
             return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);
-        return pipe_launch<128, 128, 64, 2, false, false, true>(p, silu, stream);
+        return pipe_wide<true>(p, xf, w8, silu, stream);
     }
     Kern k = pick_kernel<BM, true>(xf, w8, silu, p.after.count != 0);
     hipLaunchKernelGGL(k, dim3(gx, gy), dim3(kThreads), 0, (hipStream_t)stream, p);
@@ -956,10 +1046,14 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
 
 extern "C" size_t tessera_hip_linear_workspace(const ts_linear_args *a) {
     if (!a) return 0;
-    return a->m <= 64 ? tessera_hip_lanes_workspace(a) : 0;
+    if (a->m <= 64) return tessera_hip_lanes_workspace(a);
+    if (ts::block_form(a->w_dtype) || a->n < 1 || a->k < 64 || !pipe_fits(0, a->k, 4)) return 0;
+    const uint32_t splits = plan_split(a).splits;
+    const bool pair = (a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS;
+    return splits <= 1 ? 0 : (size_t)splits * a->m * a->n * (pair ? 2 : 1) * sizeof(float);
 }
 
 extern "C" int tessera_hip_linear(const ts_linear_args *a, void *stream) {
     TS_REQUIRE(a, "linear: null args");
-    return a->m <= 64 ? tessera_hip_lanes(a, stream) : tessera_hip_tiled(a, stream);
+    return a->m <= 64 ? tessera_hip_lanes(a, stream) : tiled(a, true, stream);
 }

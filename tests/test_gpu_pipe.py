@@ -105,3 +105,40 @@ def test_pipe_picked(x, w, silu, counts):
         g, u = full[:, :n], full[:, n:]
         want = g / (1 + np.exp(-g)) * u
         assert np.all(np.abs(got[sel] - want) <= 1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5), f"matrix {e}"
+
+
+@pytest.mark.parametrize("x,w", FORMS + [("bf16", "bf16")])
+@pytest.mark.parametrize("m,n,k,pair", [(65, 64, 4096, False), (100, 130, 4160, False), (129, 33, 2048, True),
+                                        (700, 700, 6144, False)])
+def test_pipe_split_k(m, n, k, pair, x, w):
+    """Few tiles and a deep k: split across groups (64 x 64 and 128 x 128 tiles, ragged columns,
+    a step count the splits do not divide), the sums finished by the second kernel; the same
+    product without the workspace runs unsplit."""
+    import ctypes as C
+
+    from tessera_amd import abi, rules as R
+    if w == "e4m3":
+        k = k // 128 * 128
+    r = rng(m + n)
+    O.set_threads(O.lib().or_threads_available())
+    xd, wd, sd, xf, wf, full = operands(r, m, 2 * n if pair else n, k, x, w)
+    O.set_threads(1)
+    bound = linear_bound(xf, wf)
+    if pair:
+        g, u, bg, bu = full[:, :n], full[:, n:], bound[:, :n], bound[:, n:]
+        want = O.act("silu", g) * u
+        bound = 1.1 * bg * np.abs(u) + np.abs(g) * bu + 1e-5
+    else:
+        want = full
+    out = torch.empty((m, n), device="cuda")
+    a = R.linear_args(xd, wd, out, w_scale=sd, stages=abi.TS_AFTER_SILU_MUL if pair else 0)
+    assert abi.load().tessera_hip_linear_workspace(C.byref(a)) > 0
+    got = from_dev(R.linear(xd, wd, w_scale=sd, silu_mul=pair))
+    assert np.all(np.abs(got.astype(np.float64) - want) <= bound)
+    res = r.standard_normal((m, n)).astype(np.float32)
+    added = from_dev(R.linear(xd, wd, w_scale=sd, silu_mul=pair, a0=to_dev(res, torch)))
+    assert np.array_equal(added, got + res)
+    got16 = from_dev(R.linear(xd, wd, w_scale=sd, silu_mul=pair, out_dtype=torch.bfloat16))
+    assert np.array_equal(got16, O.bf16_widen(O.bf16_narrow(got)))
+    abi.call("tessera_hip_linear", C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert np.all(np.abs(from_dev(out).astype(np.float64) - want) <= bound)
