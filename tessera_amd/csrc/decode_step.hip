@@ -30,6 +30,8 @@
 // poll that passes 2 s (100 MHz clock) sets the error word; every poll also watches
 // that word, and a failed poll lets its group run on without waiting, so the grid
 // always ends. Groups are launched cooperatively (all resident), one per CU.
+#include <type_traits>
+
 #include <string.h>
 
 #include <algorithm>
@@ -678,15 +680,18 @@ TS_DEV void att_role(const DecodeStepArgs &p, Ctx &c, const Hand &hd, uint32_t h
         for (uint32_t l = 0; l < p.L; l++) {
             const uint16_t *kc = p.k_cache[l], *vc = p.v_cache[l];
             // Kept rows of earlier positions: this wave's first kPre blocks, now.
-            u32x4 kk[kPre], vv[kPre];
+            auto rows_of = [&](uint32_t i0, u32x4 (&kq)[kPre], u32x4 (&vq)[kPre]) {
 #pragma unroll
-            for (int i = 0; i < kPre; i++) {
-                const uint32_t key = min(4 * (wave + kW * i) + kr, last);
-                const uint64_t row = ((uint64_t)c.tbl[key >> shift] << shift) | (key & mask);
-                const size_t e = (row * Hkv + a) * 128 + 8 * part;
-                kk[i] = *(const u32x4 *)(kc + e);
-                vv[i] = *(const u32x4 *)(vc + e);
-            }
+                for (int i = 0; i < kPre; i++) {
+                    const uint32_t key = min(4 * (wave + kW * (i0 + i)) + kr, last);
+                    const uint64_t row = ((uint64_t)c.tbl[key >> shift] << shift) | (key & mask);
+                    const size_t e = (row * Hkv + a) * 128 + 8 * part;
+                    kq[i] = *(const u32x4 *)(kc + e);
+                    vq[i] = *(const u32x4 *)(vc + e);
+                }
+            };
+            u32x4 kk[kPre], vv[kPre];
+            rows_of(0, kk, vv);
             float ga = 0.0f, gb = 0.0f;
             if (wave == 0) { ga = p.q_norm[l][lane]; gb = p.q_norm[l][lane + 64]; }
             if (wave == 1) { ga = p.k_norm[l][lane]; gb = p.k_norm[l][lane + 64]; }
@@ -726,30 +731,26 @@ TS_DEV void att_role(const DecodeStepArgs &p, Ctx &c, const Hand &hd, uint32_t h
 #pragma unroll
             for (int e = 0; e < 8; e++) o[e] = 0.0f;
 
-            for (uint32_t i0 = 0; i0 < mine; i0 += kPre) {
-                if (i0) {  // contexts past kW kPre blocks: load this pass now
-#pragma unroll
-                    for (int i = 0; i < kPre; i++) {
-                        const uint32_t key = min(4 * (wave + kW * (i0 + i)) + kr, last);
-                        const uint64_t row = ((uint64_t)c.tbl[key >> shift] << shift) | (key & mask);
-                        const size_t e = (row * Hkv + a) * 128 + 8 * part;
-                        kk[i] = *(const u32x4 *)(kc + e);
-                        vv[i] = *(const u32x4 *)(vc + e);
-                    }
-                }
+            // One pass of kPre blocks from block i0 of this wave. EDGE: a key of the pass may be
+            // pos (whose row is the new one) or past it; else no value is tested or replaced,
+            // the same arithmetic (a third of a pass's vector instructions, which are what a
+            // long context costs: a step at 1000 keys 669 -> 608 us, at 2000 959 -> 804).
+            auto pass = [&](uint32_t i0, const u32x4 (&kq)[kPre], const u32x4 (&vq)[kPre], auto edge) {
+#pragma clang fp contract(off)  // each rounding as written: both forms give the same bits
+                constexpr bool EDGE = decltype(edge)::value;
                 float sc[kPre];
                 bool ok[kPre];
 #pragma unroll
                 for (int i = 0; i < kPre; i++) {
                     const uint32_t key = 4 * (wave + kW * (i0 + i)) + kr;
-                    ok[i] = key <= pos;
-                    const u32x4 kv = key == pos ? knew : kk[i];
+                    ok[i] = !EDGE || key <= pos;
+                    const u32x4 kv = EDGE && key == pos ? knew : kq[i];
                     const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w};
                     float s0 = 0.0f;
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        s0 += q[2 * e] * lo_bf16(kw[e]);
-                        s0 += q[2 * e + 1] * hi_bf16(kw[e]);
+                        s0 = fmaf(q[2 * e], lo_bf16(kw[e]), s0);
+                        s0 = fmaf(q[2 * e + 1], hi_bf16(kw[e]), s0);
                     }
                     sc[i] = ok[i] ? row16_sum(s0) * sl2 : -INFINITY;
                 }
@@ -765,19 +766,40 @@ TS_DEV void att_role(const DecodeStepArgs &p, Ctx &c, const Hand &hd, uint32_t h
                 for (int i = 0; i < kPre; i++) {
                     const float pk = ok[i] ? __builtin_amdgcn_exp2f(sc[i] - mn) : 0.0f;
                     sum += pk;
-                    const u32x4 vx = (4 * (wave + kW * (i0 + i)) + kr) == pos ? vnew : vv[i];
+                    const u32x4 vx = EDGE && (4 * (wave + kW * (i0 + i)) + kr) == pos ? vnew : vq[i];
                     const uint32_t vw[4] = {ok[i] ? vx.x : 0u, ok[i] ? vx.y : 0u, ok[i] ? vx.z : 0u,
                                             ok[i] ? vx.w : 0u};
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        acc[2 * e] += pk * lo_bf16(vw[e]);
-                        acc[2 * e + 1] += pk * hi_bf16(vw[e]);
+                        acc[2 * e] = fmaf(pk, lo_bf16(vw[e]), acc[2 * e]);
+                        acc[2 * e + 1] = fmaf(pk, hi_bf16(vw[e]), acc[2 * e + 1]);
                     }
                 }
-                ls = ls * alpha + rows4_sum(sum);
+                ls = fmaf(ls, alpha, rows4_sum(sum));
                 m = mn;
 #pragma unroll
-                for (int e = 0; e < 8; e++) o[e] = o[e] * alpha + acc[e];
+                for (int e = 0; e < 8; e++) o[e] = fmaf(o[e], alpha, acc[e]);
+            };
+            if (mine <= kPre) {
+                pass(0, kk, vv, std::true_type());
+            } else {
+                // Passes that end before pos, their next pass's rows on the way while they
+                // compute; the last one or two meet pos.
+                u32x4 kb[kPre], vb[kPre];
+                uint32_t i0 = 0;
+                for (; i0 + kPre < mine && 4 * (wave + kW * (i0 + kPre - 1)) + 3 < pos; i0 += kPre) {
+                    rows_of(i0 + kPre, kb, vb);
+                    pass(i0, kk, vv, std::false_type());
+#pragma unroll
+                    for (int i = 0; i < kPre; i++) {
+                        kk[i] = kb[i];
+                        vv[i] = vb[i];
+                    }
+                }
+                for (; i0 < mine; i0 += kPre) {
+                    pass(i0, kk, vv, std::true_type());
+                    if (i0 + kPre < mine) rows_of(i0 + kPre, kk, vv);
+                }
             }
 #ifdef TS_FINE
             mark(p, c, t, l, 3);
