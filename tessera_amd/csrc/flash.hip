@@ -528,8 +528,13 @@ __global__ __launch_bounds__(256 * HG) void flash_rows_kernel(FlashParams p) {
 }
 
 int flash_launch(const FlashParams &p, bool f32, void *stream, const char *rule) {
-    // Two q heads per group when the kv heads are shared in pairs (or more, evenly).
-    const int hg = (p.heads / p.kv_heads) % 2 == 0 ? 2 : 1;
+    // Two q heads per group when the kv heads are shared in pairs (or more, evenly) and the
+    // pairs alone give more than half the CUs a group; below that, with f32 q, a head a group puts one
+    // wave on a SIMD where two waited on each other's softmax (one prompt of 1000, 16 heads over
+    // 8, 88 -> 66 us, of 2000 150 -> 115; bf16 q 47.5 -> 44.4, but windowed ones lose 1%), the same
+    // bits.
+    const uint32_t pairs = (p.rows + kRows - 1) / kRows * (p.heads / 2);
+    const int hg = (p.heads / p.kv_heads) % 2 == 0 && (pairs > 128 || !f32) ? 2 : 1;
     const auto kern = hg == 2 ? (f32 ? flash_rows_kernel<true, 2> : flash_rows_kernel<false, 2>)
                               : (f32 ? flash_rows_kernel<true, 1> : flash_rows_kernel<false, 1>);
     // The key blocks' dynamic LDS, raised once per process (thread-safe static
