@@ -851,9 +851,10 @@ Kern pick_kernel(bool xf, bool w8, bool silu, bool chain) {
 namespace {
 
 // The k split of a product of more than 64 rows whose tiles alone leave CUs idle: times in
-// us, from what the pipelined tiles take a 64-deep step (64 x 64 0.4, f32 rows 0.5 with one
-// group a CU and 0.7 with two; 128 x 128 0.9 and 1.7) and what the second kernel takes (4 us and
-// its sums' way to memory and back at 5 TB/s); a split has to promise 15%. Measured: 128 f32 rows by 1024 x 3072 23.8 -> 11.6
+// us, from what the pipelined tiles take a 64-deep step with one group a CU and with two (64 x
+// 64 0.4, f32 rows 0.5 and 0.7; 128 x 128 0.55 and 0.9, f32 rows 1.0 and 1.7) and what the
+// second kernel takes (4 us and its sums' way to memory and back at 5 TB/s); a split has to
+// promise 15%. Measured: 128 f32 rows by 1024 x 3072 23.8 -> 11.6
 // us, 300 bf16 rows by e4m3 4096 x 14336 69 -> 52, 500 by bf16 2560 x 9728 59 -> 40, 1200 f32 rows
 // by 2048 x 8192 129 -> 91; 1000 f32 rows by 1024 x 3072 24.8 against 26.8 split in two.
 struct Split {
@@ -867,9 +868,12 @@ Split plan_split(const ts_linear_args *a) {
     Split best = {1, false};
     auto tiles = [&](uint32_t t) { return (uint64_t)((a->n + (pair ? t / 2 : t) - 1) / (pair ? t / 2 : t)) * ((a->m + t - 1) / t); };
     const float sums = 8e-6f / 5 * (float)a->m * (float)a->n * (pair ? 2 : 1);
+    auto step_us = [&](bool wide, bool shared) {
+        return wide ? (xf ? (shared ? 1.7f : 1.0f) : shared ? 0.9f : 0.55f) : !xf ? 0.4f : shared ? 0.7f : 0.5f;
+    };
     auto cost = [&](bool wide, uint32_t s) {
         const uint64_t rounds = (tiles(wide ? 128 : 64) * s + 511) / 512;
-        return (float)rounds * ((steps + s - 1) / s + 1) * (wide ? (xf ? 1.7f : 0.9f) : !xf ? 0.4f : tiles(64) * s > 256 ? 0.7f : 0.5f) + (s > 1 ? 4.0f + (s + 1) * sums : 0.0f);
+        return (float)rounds * ((steps + s - 1) / s + 1) * step_us(wide, tiles(wide ? 128 : 64) * s > 256) + (s > 1 ? 4.0f + (s + 1) * sums : 0.0f);
     };
     if (tiles(64) > 1024) return best;  // enough tiles of some size
     float least = 0.85f * cost(tiles(128) >= 256, 1);
