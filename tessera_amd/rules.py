@@ -12,6 +12,7 @@ a call into libtessera_hip.so through ``tessera_amd.abi``. Errors raise
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import torch
 
@@ -31,8 +32,10 @@ def _stream():
 
 
 class Workspace:
-    """Caller-owned scratch for split-K / split-KV partials: grown on demand, zeroed
-    once when (re)allocated (the kernels return their counters to zero)."""
+    """Scratch of one thread's calls: a new tensor for each call, so that calls on several
+    streams or threads share none (the allocator's cache keeps it in stream order, and a call
+    that is being captured gets it from the graph's own memory). Not cleared: the kernels write
+    what they read. `buf` is the last one (the routing of a picked product can be read there)."""
 
     def __init__(self, device="cuda"):
         self.device = device
@@ -41,19 +44,20 @@ class Workspace:
     def get(self, nbytes: int):
         if nbytes == 0:
             return None, 0
-        if self.buf is None or self.buf.numel() < nbytes:
-            self.buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=self.device)
-        return C.c_void_p(self.buf.data_ptr()), self.buf.numel()
+        self.buf = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        return self.buf.data_ptr(), nbytes
 
 
-_ws = {}
+_ws = threading.local()
 
 
 def workspace(device) -> Workspace:
+    """The calling thread's."""
     key = str(device)
-    if key not in _ws:
-        _ws[key] = Workspace(device)
-    return _ws[key]
+    ws = _ws.__dict__.get(key)
+    if ws is None:
+        ws = _ws.__dict__[key] = Workspace(device)
+    return ws
 
 
 BLOCK_FORMS = {"q8_0": abi.TS_Q8_0, "mxfp8": abi.TS_MXFP8, "int4_g32": abi.TS_INT4_G32, "q4_0": abi.TS_Q4_0,
@@ -119,8 +123,6 @@ def _linear(fn: str, x, w, *, out=None, out_dtype=torch.float32, w_scale=None, g
     if m > 4:  # the products of fewer rows take no workspace
         need = abi.workspace_of(fn, a)
         if need:
-            # The split sums' scratch is the call's own (the allocator's cache keeps it in stream
-            # order), so products on several streams or threads do not share it.
             scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
             a.workspace, a.workspace_bytes = scratch.data_ptr(), need
     abi.call(fn, C.byref(a), _stream())
@@ -237,19 +239,16 @@ def moe_layer(h, router, w_in, w_out, *, top=8, shared_in=None, shared_out=None,
 
 
 def rows_args(q, k, v, out, slots, positions, *, keys, scale, table=None, kept_pages=0, page=16,
-              back=abi.U32_MAX, max_position=None, status=None):
-    rows, heads, width = q.shape
-    a = abi.RowsArgs()
-    a.q, a.k, a.v, a.out = _ptr(q), _ptr(k), _ptr(v), _ptr(out)
-    a.slots, a.positions, a.kept_table = _ptr(slots), _ptr(positions), _ptr(table)
-    a.rows, a.keys, a.heads, a.kv_heads, a.width = rows, keys, heads, k.shape[-2], width
-    a.back, a.kept_pages, a.page, a.scale = back, kept_pages, page, scale
-    a.q_dtype, a.kv_dtype, a.out_dtype = _DT[q.dtype], _DT[k.dtype], _DT[out.dtype]
+              back=abi.U32_MAX, max_position=None, status=None, shape=None):
+    # attend_step, whose q is in its product rows, passes the shape in place of q
+    rows, heads, width = shape or q.shape
     if max_position is None:
         max_position = int(positions.max().item()) if rows else 0
-    a.max_position = max_position
-    a.status = _ptr(status)  # int32 device word: TS_STATUS_* bits of refused rows
-    return a
+    # status: int32 device word, TS_STATUS_* bits of refused rows
+    return abi.RowsArgs(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(slots), _ptr(positions), _ptr(table), None, 0, rows,
+                        keys, heads, k.shape[-2], width, back, kept_pages, page, scale,
+                        abi.TS_F32 if q is None else _DT[q.dtype], _DT[k.dtype], _DT[out.dtype], max_position,
+                        _ptr(status))
 
 
 def attend_rows(q, k, v, slots, positions, *, keys, scale, table=None, kept_pages=0, page=16,
@@ -280,9 +279,8 @@ def attend_step(qkv, q_gain, k_gain, k, v, slots, positions, *, heads, keys, sca
         angles = rope_table(keys, theta, device=qkv.device)
     if out is None:
         out = torch.empty((rows, heads, 128), dtype=torch.float32, device=qkv.device)
-    qshape = torch.empty((rows, heads, 128), device=qkv.device)  # shape carrier only
-    a = rows_args(qshape, k, v, out, slots, positions, keys=keys, scale=scale, table=table,
-                  kept_pages=kept_pages, page=page, back=back, max_position=max_position)
+    a = rows_args(None, k, v, out, slots, positions, keys=keys, scale=scale, table=table, kept_pages=kept_pages,
+                  page=page, back=back, max_position=max_position, shape=(rows, heads, 128))
     need = abi.load().tessera_hip_attend_rows_workspace(C.byref(a))
     a.workspace, a.workspace_bytes = workspace(qkv.device).get(need)
     st = abi.StepArgs(a, _ptr(qkv), _ptr(q_gain), _ptr(k_gain), _ptr(angles), angles.shape[0], eps)
