@@ -612,12 +612,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     // Stage s has landed once no more than the later stages' loads are outstanding; the
     // barrier also ends every wave's reads of the stage refilled next. The steps that refill
-    // run without a test of what is left.
-    uint32_t s = 0, at = 0, fill = NS - 1;  // the slots of this step and of the stage loaded in it
-    for (; s + NS - 1 < steps; s++) {
+    // run without a test of what is left, a ring's worth of them unrolled: a step's slot is a
+    // constant. With stages to spare (NS > 2) the refill is issued behind the matrix work,
+    // where its writes to LDS do not meet the step's reads; with two stages it has only this
+    // step to land in. 2048 bf16 rows by 1024 x 3072 22.0 -> 20.4 us (64 x 64 tiles; unrolled
+    // alone 21.2, the form before buffer loads 21.5), by 2 x 3072 x 1024 32.9 -> 32.1 (128 x 192); two stages refilled late: 1000
+    // by 4096 x 4096 41 -> 55. Not where a step's own registers are many, which unrolled got
+    // slower: f32 rows by e4m3 on 128 x 128 (1000 by 4096 x 14336 231 -> 246), f32 rows
+    // by bf16 picked (4096 rows by 32 matrices of 2 x 1024 x 2048 133 -> 135).
+    constexpr bool UNROLL = !XF32 || (PICK ? W8 : NS > 2), LATE = UNROLL && NS > 2;
+    auto refilling = [&](uint32_t s, uint32_t at, uint32_t fill) {
         pipe_wait<(P::NA + P::NB) * (NS - 2)>();
-        fetch(fill, (s0 + s + NS - 1) * KD);
+        if (!LATE) fetch(fill, (s0 + s + NS - 1) * KD);
         multiply(at);
+        if (LATE) fetch(fill, (s0 + s + NS - 1) * KD);
+    };
+    uint32_t s = 0;
+    if (UNROLL)
+        for (; s + 2 * NS - 2 < steps; s += NS)
+#pragma unroll
+            for (int u = 0; u < NS; u++) refilling(s + u, u, (u + NS - 1) % NS);
+    uint32_t at = 0, fill = NS - 1;  // the slots of this step and of the stage loaded in it
+    for (; s + NS - 1 < steps; s++) {
+        refilling(s, at, fill);
         at = at == NS - 1 ? 0 : at + 1;
         fill = fill == NS - 1 ? 0 : fill + 1;
     }

@@ -51,6 +51,21 @@ def test_pipe_edges(m, n, k, x, w):
     assert np.array_equal(got16, O.bf16_widen(O.bf16_narrow(got32)))
 
 
+@pytest.mark.parametrize("x,w", FORMS + [("bf16", "bf16")])
+@pytest.mark.parametrize("m,n,most", [(66, 30, 12), (1030, 4100, 6)])
+def test_pipe_step_counts(m, n, most, x, w):
+    """Every count of k steps around the ring: none that refills a stage, some, whole turns of
+    the ring and what is left behind them, on 64 x 64 and 128-wide tiles."""
+    from tessera_amd import rules as R
+    r = rng(m + most)
+    O.set_threads(O.lib().or_threads_available())
+    for steps in range(1, most + 1):
+        xd, wd, sd, xf, wf, want = operands(r, m, n, 64 * steps, x, w)
+        got = from_dev(R.tiled(xd, wd, w_scale=sd))
+        assert np.all(np.abs(got.astype(np.float64) - want) <= linear_bound(xf, wf)), f"{steps} steps"
+    O.set_threads(1)
+
+
 @pytest.mark.parametrize("x,w", FORMS)
 @pytest.mark.parametrize("m,n,k", [(70, 40, 128), (1030, 2050, 64)])
 def test_pipe_gate_up(m, n, k, x, w):
