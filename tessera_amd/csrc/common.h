@@ -90,8 +90,8 @@ struct Route {
     uint32_t *perm;        // [rows]: row at each sorted position
 };
 size_t route_words(uint32_t rows, uint32_t count);
-int route_launch(const uint32_t *ids, uint32_t rows, uint32_t first, uint32_t count, uint32_t tile_rows, void *ws,
-                 Route *route, void *stream);
+int route_launch(const uint32_t *ids, uint32_t rows, uint32_t first, uint32_t count, uint32_t tile_rows,
+                 uint32_t few_most, void *ws, Route *route, void *stream);
 // Rows whose id is outside the set: their sum is 0, stored through the chain.
 int zero_absent_launch(const Route &route, uint32_t count, void *out, uint32_t n, int out_bf16, const ts_after &after,
                        void *stream);

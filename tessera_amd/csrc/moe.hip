@@ -39,6 +39,11 @@ __global__ __launch_bounds__(kChunk) void route_count(const uint32_t *ids, uint3
     for (uint32_t b = threadIdx.x; b < B; b += kChunk) offs[(size_t)blockIdx.x * B + b] = hist[b];
 }
 
+// Row tiles of a matrix of r rows: tile_rows each, or 32 where it has at most few_most.
+TS_DEV uint32_t row_tiles(uint32_t r, uint32_t tile_rows, uint32_t few_most) {
+    return r <= few_most ? (r + 31) / 32 : (r + tile_rows - 1) / tile_rows;
+}
+
 // Exclusive scan of per-thread segment sums held in part[kScan] (in place).
 TS_DEV void scan_parts(uint32_t *part) {
     __syncthreads();
@@ -56,7 +61,8 @@ TS_DEV void scan_parts(uint32_t *part) {
 // One group: per bucket, chunk counts -> positions within the bucket; bucket totals
 // -> row_start; row tiles per matrix -> tile_start; then positions made absolute.
 __global__ __launch_bounds__(kScan) void route_scan(uint32_t *offs, uint32_t chunks, uint32_t rows, uint32_t count,
-                                                    uint32_t tile_rows, uint32_t *row_start, uint32_t *tile_start) {
+                                                    uint32_t tile_rows, uint32_t few_most, uint32_t *row_start,
+                                                    uint32_t *tile_start) {
     __shared__ uint32_t part[kScan], tpart[kScan];
     const uint32_t B = count + 1, t = threadIdx.x;
     const uint32_t per = (B + kScan - 1) / kScan, b0 = t * per, b1 = min(B, b0 + per);
@@ -80,7 +86,7 @@ __global__ __launch_bounds__(kScan) void route_scan(uint32_t *offs, uint32_t chu
         }
         row_start[b] = s;  // total for now
         seg += s;
-        tseg += b < count ? (s + tile_rows - 1) / tile_rows : 0;
+        tseg += b < count ? row_tiles(s, tile_rows, few_most) : 0;
     }
     part[t] = seg;
     tpart[t] = tseg;
@@ -100,7 +106,7 @@ __global__ __launch_bounds__(kScan) void route_scan(uint32_t *offs, uint32_t chu
         }
         if (b < count) {
             tile_start[b] = tbase;
-            tbase += (tot + tile_rows - 1) / tile_rows;
+            tbase += row_tiles(tot, tile_rows, few_most);
         }
         base += tot;
     }
@@ -129,8 +135,8 @@ TS_DEV uint32_t wave_scan(uint32_t v, uint32_t lane) {
 constexpr uint32_t kFastWaves = kScan / 64, kFastCW = 8, kFastBS = 5;
 constexpr uint32_t kFastChunks = kFastWaves * kFastCW, kFastBuckets = 64 * kFastBS;
 __global__ __launch_bounds__(kScan) void route_scan_fast(uint32_t *offs, uint32_t chunks, uint32_t rows,
-                                                         uint32_t count, uint32_t tile_rows, uint32_t *row_start,
-                                                         uint32_t *tile_start) {
+                                                         uint32_t count, uint32_t tile_rows, uint32_t few_most,
+                                                         uint32_t *row_start, uint32_t *tile_start) {
     __shared__ uint32_t wsum[kFastWaves][kFastBuckets], tot_s[kFastBuckets], base_s[kFastBuckets];
     const uint32_t B = count + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t v[kFastBS][kFastCW];
@@ -169,7 +175,7 @@ __global__ __launch_bounds__(kScan) void route_scan_fast(uint32_t *offs, uint32_
             const uint32_t b = lane * kPer + i;
             if (b < B) {
                 rs += tot_s[b];
-                ts += b < count ? (tot_s[b] + tile_rows - 1) / tile_rows : 0;
+                ts += b < count ? row_tiles(tot_s[b], tile_rows, few_most) : 0;
             }
         }
         uint32_t rb = wave_scan(rs, lane) - rs, tb = wave_scan(ts, lane) - ts;
@@ -180,7 +186,7 @@ __global__ __launch_bounds__(kScan) void route_scan_fast(uint32_t *offs, uint32_
                 row_start[b] = rb;
                 if (b < count) tile_start[b] = tb;
                 rb += tot_s[b];
-                tb += b < count ? (tot_s[b] + tile_rows - 1) / tile_rows : 0;
+                tb += b < count ? row_tiles(tot_s[b], tile_rows, few_most) : 0;
             }
         }
         if (lane == 63) {
@@ -315,8 +321,8 @@ size_t route_words(uint32_t rows, uint32_t count) {
     return chunks * B + (B + 1) + ((size_t)count + 1) + rows;
 }
 
-int route_launch(const uint32_t *ids, uint32_t rows, uint32_t first, uint32_t count, uint32_t tile_rows, void *ws,
-                 Route *route, void *stream) {
+int route_launch(const uint32_t *ids, uint32_t rows, uint32_t first, uint32_t count, uint32_t tile_rows,
+                 uint32_t few_most, void *ws, Route *route, void *stream) {
     const uint32_t chunks = (rows + kChunk - 1) / kChunk, B = count + 1;
     uint32_t *offs = (uint32_t *)ws;
     route->row_start = offs + (size_t)chunks * B;
@@ -327,10 +333,10 @@ int route_launch(const uint32_t *ids, uint32_t rows, uint32_t first, uint32_t co
                        offs);
     if (chunks <= kFastChunks && B <= kFastBuckets)
         hipLaunchKernelGGL(route_scan_fast, dim3(1), dim3(kScan), 0, s, offs, chunks, rows, count, tile_rows,
-                           route->row_start, route->tile_start);
+                           few_most, route->row_start, route->tile_start);
     else
         hipLaunchKernelGGL(route_scan, dim3(1), dim3(kScan), 0, s, offs, chunks, rows, count, tile_rows,
-                           route->row_start, route->tile_start);
+                           few_most, route->row_start, route->tile_start);
     hipLaunchKernelGGL(route_place, dim3(chunks), dim3(kChunk), 0, s, ids, rows, first, count, offs, route->perm);
     TS_CHECK_LAUNCH("picked routing");
     return TS_OK;

@@ -56,6 +56,7 @@ struct TiledParams {
     uint32_t splits;     // pipelined tiles: groups along k; more than 1: raw sums to part
     float *part;         // [split][gate, up or one][m][n]
     uint32_t pick_cols;  // PICK on the pipelined tiles: column tiles (0: a 2-D grid of them)
+    uint32_t few_most;   // PICK: matrices of up to this many rows run as 32-row tiles
 };
 
 // Byte offset of (row, chunk) in a swizzled [rows][8 chunks of 16B] tile.
@@ -411,13 +412,19 @@ TS_DEV void pipe_wait_ahead(uint32_t ahead) {
 // x 64 tiles only: larger ones would spill), or raw sums of a split of k to memory.
 enum Ends { kPlain, kChain, kSplit };
 
-template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END>
+// Stages of the 32-row tiles (16 to 24 KiB each).
+template <bool XF32>
+constexpr int kFewStages = XF32 ? 3 : 4;
+
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END, bool ROLL>
+TS_DEV void pipe_tile(const TiledParams &p, char *lds, uint32_t n0, uint32_t m0, uint32_t mend, const char *w,
+                      const uint16_t *scale, uint32_t split);
+
+// FEW (picked products): the matrices of at most p.few_most rows run as 32-row tiles. ROLL: the
+// steps are unrolled (not in a FEW kernel, whose two forms share the instruction cache).
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END, bool FEW>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tiled_pipe_kernel(TiledParams p) {
-    using P = Pipe<TM, TN, KD, NS, XF32, W8>;
     extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: two groups share a CU
-    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t wm = wave / P::GN, wn = wave % P::GN;
-    const uint32_t col = lane & 15, grp = lane >> 4;
     constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
     uint32_t tx = blockIdx.x, ty = blockIdx.y, split = 0;
     if (!PICK) {
@@ -482,12 +489,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             else hi = mid;
         }
         const uint32_t e = lo;
-        m0 = p.row_start[e] + (y - p.tile_start[e]) * TM;
-        mend = p.row_start[e + 1];
         const size_t first_row = (size_t)e * p.stride + p.offset;
         w += first_row * p.k * (W8 ? 1 : 2);
         if (W8) scale += first_row;
+        mend = p.row_start[e + 1];
+        if constexpr (FEW)
+            if (mend - p.row_start[e] <= p.few_most)
+                return pipe_tile<32, TN, 64, kFewStages<XF32>, XF32, W8, SILU, PICK, END, false>(
+                    p, lds, n0, p.row_start[e] + (y - p.tile_start[e]) * 32, mend, w, scale, split);
+        m0 = p.row_start[e] + (y - p.tile_start[e]) * TM;
     }
+    pipe_tile<TM, TN, KD, NS, XF32, W8, SILU, PICK, END, !FEW>(p, lds, n0, m0, mend, w, scale, split);
+}
+
+// The tile of rows [m0, min(m0 + TM, mend)) and of the columns from n0 on.
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END, bool ROLL>
+TS_DEV void pipe_tile(const TiledParams &p, char *lds, uint32_t n0, uint32_t m0, uint32_t mend, const char *w,
+                      const uint16_t *scale, uint32_t split) {
+    using P = Pipe<TM, TN, KD, NS, XF32, W8>;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / P::GN, wn = wave % P::GN;
+    const uint32_t col = lane & 15, grp = lane >> 4;
+    constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
     // PICK: the output row of tile row tr (~0u past the matrix's rows), read where needed
     // (no LDS copy, so two groups' stages fill a CU's LDS).
     auto row_out = [&](uint32_t tr) { return m0 + tr < mend ? p.perm[m0 + tr] : 0xffffffffu; };
@@ -620,7 +643,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // by 4096 x 4096 41 -> 55. Not where a step's own registers are many, which unrolled got
     // slower: f32 rows by e4m3 on 128 x 128 (1000 by 4096 x 14336 231 -> 246), f32 rows
     // by bf16 picked (4096 rows by 32 matrices of 2 x 1024 x 2048 133 -> 135).
-    constexpr bool UNROLL = !XF32 || (PICK ? W8 : NS > 2), LATE = UNROLL && NS > 2;
+    constexpr bool UNROLL = ROLL && (!XF32 || (PICK ? W8 : NS > 2)), LATE = UNROLL && NS > 2;
     auto refilling = [&](uint32_t s, uint32_t at, uint32_t fill) {
         pipe_wait<(P::NA + P::NB) * (NS - 2)>();
         if (!LATE) fetch(fill, (s0 + s + NS - 1) * KD);
@@ -777,16 +800,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 }
 
-template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool PICK, Ends END = kPlain>
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool PICK, Ends END = kPlain, bool FEW = false>
 int pipe_launch(TiledParams p, bool silu, void *stream) {
-    constexpr int lds = Pipe<TM, TN, KD, NS, XF32, W8>::LDS;
-    const void *k = silu ? (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END>
-                         : (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END>;
+    constexpr int lds = [] {
+        constexpr int own = Pipe<TM, TN, KD, NS, XF32, W8>::LDS;
+        if constexpr (FEW) return std::max(own, Pipe<32, TN, 64, kFewStages<XF32>, XF32, W8>::LDS);
+        return own;
+    }();
+    const void *k = silu ? (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END, FEW>
+                         : (const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END, FEW>;
     // The dynamic LDS size is raised once per kernel (thread-safe static initialisation).
     static const hipError_t attr[2] = {
-        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END>,
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, false, PICK, END, FEW>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END>,
+        hipFuncSetAttribute((const void *)tiled_pipe_kernel<TM, TN, KD, NS, XF32, W8, true, PICK, END, FEW>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds)};
     if (attr[silu]) return ts::hip_status(attr[silu], "tiled (pipelined): LDS attribute");
     const uint32_t oc = silu ? TN / 2 : TN;
@@ -794,7 +821,8 @@ int pipe_launch(TiledParams p, bool silu, void *stream) {
     dim3 grid;
     if (PICK) {
         // Row tiles: at most one partial tile per matrix beyond rows / TM full ones.
-        const uint32_t gy = (p.m + TM - 1) / TM + p.matrices;
+        constexpr uint32_t RT = FEW ? 32 : TM;
+        const uint32_t gy = (p.m + RT - 1) / RT + p.matrices;
         // XCD-aware (C5 gate/up 1214 -> 1189 us, layer 2.48-2.53 -> 2.44 ms) where the
         // one-dimensional grid fits.
         if ((uint64_t)8 * gx * ((gy + 7) / 8) < (1ull << 31)) {
@@ -832,21 +860,14 @@ int pipe_small(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) 
               : pipe_launch<64, 64, 64, 4, false, false, false, END>(p, silu, stream);
 }
 
-// 128 x 128 tiles.
-template <bool PICK, Ends END = kPlain>
+// 128 x 128 tiles. FEW: 32 x 128 for the matrices of few rows, the four waves side by side
+// along the columns.
+template <bool PICK, Ends END = kPlain, bool FEW = false>
 int pipe_wide(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
-    if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK, END>(p, silu, stream)
-                      : pipe_launch<128, 128, 32, 3, true, false, PICK, END>(p, silu, stream);
-    return w8 ? pipe_launch<128, 128, 64, 3, false, true, PICK, END>(p, silu, stream)
-              : pipe_launch<128, 128, 64, 2, false, false, PICK, END>(p, silu, stream);
-}
-
-// 32 x 128 tiles for matrices of few rows: the four waves side by side along the columns.
-int pipe_few(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
-    if (xf) return w8 ? pipe_launch<32, 128, 64, 3, true, true, true>(p, silu, stream)
-                      : pipe_launch<32, 128, 64, 3, true, false, true>(p, silu, stream);
-    return w8 ? pipe_launch<32, 128, 64, 4, false, true, true>(p, silu, stream)
-              : pipe_launch<32, 128, 64, 4, false, false, true>(p, silu, stream);
+    if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK, END, FEW>(p, silu, stream)
+                      : pipe_launch<128, 128, 32, 3, true, false, PICK, END, FEW>(p, silu, stream);
+    return w8 ? pipe_launch<128, 128, 64, 3, false, true, PICK, END, FEW>(p, silu, stream)
+              : pipe_launch<128, 128, 64, 2, false, false, PICK, END, FEW>(p, silu, stream);
 }
 
 using Kern = void (*)(TiledParams);
@@ -921,7 +942,7 @@ int tiled(const ts_linear_args *a, bool may_split, void *stream) {
                a->stages);
     TS_REQUIRE(ts::aligned(a->x, 16) && ts::aligned(a->w, 16), "tiled: x and w must be 16-byte aligned");
     TiledParams p;
-    p.pick_cols = 0;
+    p.pick_cols = p.few_most = 0;
     int rc = ts::linear_after(a, "tiled", &p.after);
     if (rc) return rc;
     const int big = ts::tiled_big_launch(a, stream);
@@ -1030,13 +1051,21 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // and a 128-row one loads its few rows 128 / rows times over beside the weights. 128
     // matrices of 4096 x 1536 at 1 / 16 rows each 213 -> 186 / 324 -> 319 us (2 x 1536 x 4096
     // 374 -> 373 / 575 -> 570: HBM), at 32 rows 350 -> 369; one token's 8 matrices 62 -> 41.
+    // A routing may still give most rows to few matrices. Where even that fits two rounds of
+    // groups, smaller tiles win (512 rows on 4 of the 128: 39 -> 33 us); past it the matrices
+    // of more than 64 rows take 128-row tiles, their weights read once for 128 rows (2048 rows
+    // on 4 matrices 67 -> 46 us, 2 x 1536 x 4096 102 -> 74; on Zipf-distributed matrices within 2%
+    // of 32-row tiles alone).
+    const uint32_t pick_gx = a->stages & TS_AFTER_SILU_MUL ? (a->n + 63) / 64 : (a->n + 127) / 128;
     const bool few = pipe && a->rows <= 16ull * a->count;
+    const uint32_t few_most = !few ? 0 : (uint64_t)a->rows * pick_gx > 32 * 1024 ? 64 : 0xffffffffu;
     ts::Route route;
-    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, few ? 32 : BM, a->workspace, &route, stream);
+    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, BM, few_most, a->workspace, &route, stream);
     if (rc) return rc;
     const bool silu = a->stages & TS_AFTER_SILU_MUL;
     TiledParams p;
     p.pick_cols = 0;
+    p.few_most = few_most;
     p.splits = 1;
     p.part = nullptr;
     p.pair_sum = 0;
@@ -1053,7 +1082,7 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // A stage chain takes the register-staged kernel (the pipelined one's chain variant spills).
     // 128 x 192 tiles where the columns divide evenly (fewer re-reads of the gathered
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
-    if (few) return pipe_few(p, xf, w8, silu, stream);
+    if (few) return pipe_wide<true, kPlain, true>(p, xf, w8, silu, stream);
     if (pipe) {
         if (!xf && !w8 && (silu ? a->n % 96 : a->n % 192) == 0)
             return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);

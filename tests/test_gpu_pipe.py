@@ -123,6 +123,33 @@ def test_pipe_picked(x, w, silu, counts):
 
 
 @pytest.mark.parametrize("x,w", FORMS + [("bf16", "bf16")])
+@pytest.mark.parametrize("silu,n,k", [(False, 136, 192), (True, 136, 192), (False, 8070, 128), (True, 4100, 128)])
+def test_pipe_picked_skewed(x, w, silu, n, k):
+    """Few rows a matrix on average, and some matrices with many: 32-row tiles, with many columns
+    128-row ones for the matrices of more than 64 rows."""
+    from tessera_amd import rules as R
+    r = rng(23 + silu)
+    count = 40
+    rows_of = {0: 161, 3: 128, 5: 65, 9: 64, 10: 33, 11: 32, 39: 1, 45: 50}
+    used = 2 * n if silu else n
+    ids = r.permutation(np.repeat(list(rows_of), list(rows_of.values()))).astype(np.uint32)
+    xd, wd, sd, xf, wf, _ = operands(r, len(ids), count * used, k, x, w)
+    got = from_dev(R.picked(xd, wd.view(count, used, k), to_dev(ids.astype(np.int32), torch), n=n, silu_mul=silu,
+                            w_scale=None if sd is None else sd.view(count, used)))
+    table = wf.reshape(count, used, k)
+    assert np.all(got[ids >= count] == 0.0)
+    for e in (e for e in rows_of if e < count):
+        sel = ids == e
+        full, b = xf[sel].astype(np.float64) @ table[e].T.astype(np.float64), linear_bound(xf[sel], table[e])
+        if not silu:
+            assert np.all(np.abs(got[sel] - full) <= b), f"matrix {e}"
+            continue
+        g, u = full[:, :n], full[:, n:]
+        assert np.all(np.abs(got[sel] - g / (1 + np.exp(-g)) * u) <=
+                      1.1 * b[:, :n] * np.abs(u) + np.abs(g) * b[:, n:] + 1e-5), f"matrix {e}"
+
+
+@pytest.mark.parametrize("x,w", FORMS + [("bf16", "bf16")])
 @pytest.mark.parametrize("m,n,k,pair", [(65, 64, 4096, False), (100, 130, 4160, False), (129, 33, 2048, True),
                                         (700, 700, 6144, False)])
 def test_pipe_split_k(m, n, k, pair, x, w):
