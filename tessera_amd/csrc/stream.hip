@@ -561,7 +561,10 @@ bool pair_of(const ts_linear_args *a) { return (a->stages & TS_AFTER_SILU_MUL) |
 // 4 in 4, 13.1 at S 1 in 16; 8 by e4m3 2 x 14336 x 4096 29.3 to 30.6 whichever.
 Plan plan_splits(const ts_linear_args *a, const Choice &c) {
     const uint32_t groups = (a->n + c.cols - 1) / c.cols, steps = (a->k + c.span - 1) / c.span;
-    const uint32_t resident = kCus * std::min(2, kMaxLds / c.lds);
+    // Two waves a SIMD: one group of 8 a CU, two of 4 where their LDS allows. (Counted by LDS
+    // alone, 8 bf16 rows by int4_g32 2 x 14336 x 4096 were split in two, 28.6 us against 23.4
+    // unsplit, and 4096 x 14336 in 14, 18.6 against 14.6 in 8.)
+    const uint32_t resident = kCus * std::min(8 * 64 / c.threads, kMaxLds / c.lds);
     const float sums = (float)a->m * a->n * (pair_of(a) ? 2 : 1) * sizeof(float);
     const float step = std::max(1.0f, c.work / 12.0f);
     Plan best = {c, 1, 1e30f};

@@ -126,6 +126,19 @@ def test_workspace_sizes():
     assert lib.tessera_hip_attend_rows_workspace(C.byref(r)) == 32 * 8 * 8 * 2 * 130 * 4
 
 
+def test_stream_splits_by_resident_groups():
+    """Block-form groups have 8 waves, two a SIMD: one group a CU whatever its LDS. 8 bf16 rows by
+    int4_g32 2 x 14336 x 4096 are 224 groups, one round unsplit; 4096 x 14336, 32 groups, is split
+    8 ways into one round."""
+    lib = abi.load()
+    a = abi.LinearArgs()
+    a.x_dtype, a.w_dtype = abi.TS_BF16, abi.TS_INT4_G32
+    a.m, a.n, a.k, a.stages = 8, 14336, 4096, abi.TS_AFTER_SILU_MUL
+    assert lib.tessera_hip_lanes_workspace(C.byref(a)) == 0
+    a.n, a.k, a.stages = 4096, 14336, 0
+    assert lib.tessera_hip_lanes_workspace(C.byref(a)) == 8 * 8 * 4096 * 4
+
+
 def test_attend_step_refuses_workspace_sized_for_attend_rows():
     """Past 2048 keys the fused step splits a span into more partitions than
     attend_rows does; a workspace that holds only attend_rows' partials is refused
