@@ -58,8 +58,10 @@ int block_gemv_launch(const ts_linear_args *a, void *stream);
 int block_tiled_launch(const ts_linear_args *a, void *stream);
 
 // 5..64 rows, weights streamed (stream.hip), arguments already checked: whether a product is
-// for it, the workspace its k split takes (without it k is not split), and the launch.
+// for it (stream_always: with any other row count too), the workspace its k split takes (a
+// smaller one holds fewer splits, none leaves k unsplit), and the launch.
 bool stream_fits(const ts_linear_args *a);
+bool stream_always(const ts_linear_args *a);
 size_t stream_workspace(const ts_linear_args *a);
 int stream_launch(const ts_linear_args *a, void *stream);
 

@@ -439,9 +439,11 @@ extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
     const Plan pl = plan(a);
     const size_t per = (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1);
     const size_t here = pl.splits <= 1 ? 0 : (size_t)pl.splits * per * sizeof(float);
-    // Never less than this file's kernel takes: fewer rows of the same product may run here,
-    // and its need grows with the rows, so the size for the most rows serves them all.
-    return ts::stream_fits(a) ? std::max(here, ts::stream_workspace(a)) : here;
+    if (!ts::stream_fits(a)) return here;
+    // Fewer rows of a small product may run in this file, which refuses less than it needs and
+    // whose need grows with the rows: the size for the most rows serves them all.
+    const size_t streamed = ts::stream_workspace(a);
+    return ts::stream_always(a) ? streamed : std::max(here, streamed);
 }
 
 extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {

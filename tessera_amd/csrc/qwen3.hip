@@ -293,14 +293,16 @@ size_t workspace_need(ts_qwen3 *m) {
     am.width = c.vocab;
     size_t need = tessera_hip_argmax_workspace(&am);
     const uint32_t H = c.hidden, D = c.head_dim;
-    const uint32_t shapes[][2] = {{(c.heads + 2 * c.kv_heads) * D, H}, {H, c.heads * D}, {c.ffn, H},
-                                  {H, c.ffn}, {c.vocab, H}};
+    const struct { uint32_t n, k, stages; } shapes[] = {{(c.heads + 2 * c.kv_heads) * D, H, TS_BEFORE_RMS_NORM},
+                                                        {H, c.heads * D, 0},
+                                                        {c.ffn, H, TS_BEFORE_RMS_NORM | TS_AFTER_SILU_MUL},
+                                                        {H, c.ffn, 0}};
     // The most split sums of any row count that a launch can carry to the few-row kernels
-    // (up to 64; fewer rows may be split more ways).
+    // (up to 64; fewer rows may be split more ways), the norm fused up to 16 rows (run_layers).
     for (uint32_t rows = 1; rows <= std::min<uint32_t>(c.max_prompt, 64); rows++)
         for (auto &sh : shapes) {
-            ts_linear_args a = lin(nullptr, nullptr, nullptr, rows, sh[0], sh[1], m);
-            if (sh[0] == c.ffn && sh[1] == H) a.stages = TS_AFTER_SILU_MUL;
+            ts_linear_args a = lin(nullptr, nullptr, nullptr, rows, sh.n, sh.k, m);
+            a.stages = rows <= 16 ? sh.stages : sh.stages & ~(uint32_t)TS_BEFORE_RMS_NORM;
             size_t w = tessera_hip_linear_workspace(&a);
             if (w > need) need = w;
         }

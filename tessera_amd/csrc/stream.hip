@@ -559,7 +559,7 @@ bool pair_of(const ts_linear_args *a) { return (a->stages & TS_AFTER_SILU_MUL) |
 // splits: 16 rows by bf16 4096 x 1536 7.7 us at S 4 unsplit, 8.8 at S 2 in 6 and S 1 in 8; 64
 // f32 rows by 2 x 3072 x 1024 14.1 us in 4 splits, 15.9 in 8; 16 by 2 x 1536 x 4096 11.7 at S
 // 4 in 4, 13.1 at S 1 in 16; 8 by e4m3 2 x 14336 x 4096 29.3 to 30.6 whichever.
-Plan plan_splits(const ts_linear_args *a, const Choice &c) {
+Plan plan_splits(const ts_linear_args *a, const Choice &c, uint32_t most) {
     const uint32_t groups = (a->n + c.cols - 1) / c.cols, steps = (a->k + c.span - 1) / c.span;
     // Two waves a SIMD: one group of 8 a CU, two of 4 where their LDS allows. (Counted by LDS
     // alone, 8 bf16 rows by int4_g32 2 x 14336 x 4096 were split in two, 28.6 us against 23.4
@@ -568,7 +568,7 @@ Plan plan_splits(const ts_linear_args *a, const Choice &c) {
     const float sums = (float)a->m * a->n * (pair_of(a) ? 2 : 1) * sizeof(float);
     const float step = std::max(1.0f, c.work / 12.0f);
     Plan best = {c, 1, 1e30f};
-    for (uint32_t s = 1; s <= std::min(steps, 32u); s++) {
+    for (uint32_t s = 1; s <= std::min(steps, most); s++) {
         const uint32_t rounds = (groups * s + resident - 1) / resident;
         const float took = (float)(rounds * ((steps + s - 1) / s + 3)) * step + (s > 1 ? 6.0f + s * sums / 1.3e6f : 0.0f);
         if (took < best.cost) {
@@ -581,60 +581,67 @@ Plan plan_splits(const ts_linear_args *a, const Choice &c) {
 
 // Block forms: S 2 up to 32 rows, else 1 (the operands of x outgrow LDS).
 template <int F, int MT>
-Plan plan_block(const ts_linear_args *a) {
+Plan plan_block(const ts_linear_args *a, uint32_t most) {
     constexpr int S = MT <= 2 ? 2 : 1;
     const bool pair = pair_of(a);
-    return plan_splits(a, a->x_dtype == TS_F32 ? (pair ? choice<F, MT, true, true, S>() : choice<F, MT, true, false, S>())
-                                               : (pair ? choice<F, MT, false, true, S>() : choice<F, MT, false, false, S>()));
+    return plan_splits(a,
+                       a->x_dtype == TS_F32 ? (pair ? choice<F, MT, true, true, S>() : choice<F, MT, true, false, S>())
+                                            : (pair ? choice<F, MT, false, true, S>() : choice<F, MT, false, false, S>()),
+                       most);
 }
 
 // bf16 and e4m3: groups of 32 (S 4), 64 or 128 columns, by the plan; S 4 only where two groups
 // still share a CU, S 2 where the operands of x fit.
 template <int F, int MT, bool XF32, bool PAIR, bool NORM>
-Plan plan_plain(const ts_linear_args *a) {
-    Plan best = plan_splits(a, choice<F, MT, XF32, PAIR, 1, NORM>());
+Plan plan_plain(const ts_linear_args *a, uint32_t most) {
+    Plan best = plan_splits(a, choice<F, MT, XF32, PAIR, 1, NORM>(), most);
     if constexpr (Shape<F, MT, XF32, PAIR, 2>::LDS <= kMaxLds) {
-        const Plan p = plan_splits(a, choice<F, MT, XF32, PAIR, 2, NORM>());
+        const Plan p = plan_splits(a, choice<F, MT, XF32, PAIR, 2, NORM>(), most);
         if (p.cost <= best.cost) best = p;
     }
     if constexpr (Shape<F, MT, XF32, PAIR, 4>::LDS <= kMaxLds / 2) {
-        const Plan p = plan_splits(a, choice<F, MT, XF32, PAIR, 4, NORM>());
+        const Plan p = plan_splits(a, choice<F, MT, XF32, PAIR, 4, NORM>(), most);
         if (p.cost <= best.cost) best = p;
     }
     return best;
 }
 
 template <int F, int MT>
-Plan plan_of(const ts_linear_args *a) {
+Plan plan_of(const ts_linear_args *a, uint32_t most) {
     if constexpr (Unit<F>::BLOCK) {
-        return plan_block<F, MT>(a);
+        return plan_block<F, MT>(a, most);
     } else {
         const bool pair = pair_of(a);
         if constexpr (MT == 1)
             if (a->stages & TS_BEFORE_RMS_NORM)
-                return pair ? plan_plain<F, 1, true, true, true>(a) : plan_plain<F, 1, true, false, true>(a);
-        return a->x_dtype == TS_F32 ? (pair ? plan_plain<F, MT, true, true, false>(a) : plan_plain<F, MT, true, false, false>(a))
-                                    : (pair ? plan_plain<F, MT, false, true, false>(a) : plan_plain<F, MT, false, false, false>(a));
+                return pair ? plan_plain<F, 1, true, true, true>(a, most) : plan_plain<F, 1, true, false, true>(a, most);
+        if (a->x_dtype == TS_F32)
+            return pair ? plan_plain<F, MT, true, true, false>(a, most) : plan_plain<F, MT, true, false, false>(a, most);
+        return pair ? plan_plain<F, MT, false, true, false>(a, most) : plan_plain<F, MT, false, false, false>(a, most);
     }
 }
 
 template <int F>
-Plan plan_rows(const ts_linear_args *a) {
+Plan plan_rows(const ts_linear_args *a, uint32_t most) {
     const uint32_t mt = (a->m + 15) / 16;
-    return mt == 1 ? plan_of<F, 1>(a) : mt == 2 ? plan_of<F, 2>(a) : mt == 3 ? plan_of<F, 3>(a) : plan_of<F, 4>(a);
+    return mt == 1 ? plan_of<F, 1>(a, most) : mt == 2 ? plan_of<F, 2>(a, most)
+         : mt == 3 ? plan_of<F, 3>(a, most) : plan_of<F, 4>(a, most);
 }
 
-Plan plan(const ts_linear_args *a) {
+constexpr uint32_t kMostSplits = 32;
+
+// most: the splits that the workspace holds.
+Plan plan(const ts_linear_args *a, uint32_t most = kMostSplits) {
     switch (a->w_dtype) {
-    case TS_Q8_0: return plan_rows<0>(a);
-    case TS_MXFP8: return plan_rows<1>(a);
-    case TS_INT4_G32: return plan_rows<2>(a);
-    case TS_Q4_0: return plan_rows<3>(a);
-    case TS_NVFP4: return plan_rows<4>(a);
-    case TS_MXFP4: return plan_rows<5>(a);
-    case TS_INT4_G128: return plan_rows<6>(a);
-    case TS_E4M3: return plan_rows<kE4M3>(a);
-    default: return plan_rows<kBf16>(a);
+    case TS_Q8_0: return plan_rows<0>(a, most);
+    case TS_MXFP8: return plan_rows<1>(a, most);
+    case TS_INT4_G32: return plan_rows<2>(a, most);
+    case TS_Q4_0: return plan_rows<3>(a, most);
+    case TS_NVFP4: return plan_rows<4>(a, most);
+    case TS_MXFP4: return plan_rows<5>(a, most);
+    case TS_INT4_G128: return plan_rows<6>(a, most);
+    case TS_E4M3: return plan_rows<kE4M3>(a, most);
+    default: return plan_rows<kBf16>(a, most);
     }
 }
 
@@ -648,10 +655,9 @@ bool fits(const ts_linear_args *a) {
            a->k % bs.block == 0 && rows * (a->k / bs.block) * bs.bytes < (1ull << 32);
 }
 
-size_t need_of(const ts_linear_args *a, const Plan &pl) {
-    if (pl.splits <= 1) return 0;
-    const size_t sums = (size_t)a->m * a->n * (pair_of(a) ? 2 : 1) + ((a->stages & TS_BEFORE_RMS_NORM) ? a->m : 0);
-    return pl.splits * sums * sizeof(float);
+// The sums of one split.
+size_t split_bytes(const ts_linear_args *a) {
+    return ((size_t)a->m * a->n * (pair_of(a) ? 2 : 1) + ((a->stages & TS_BEFORE_RMS_NORM) ? a->m : 0)) * sizeof(float);
 }
 
 }  // namespace
@@ -659,14 +665,18 @@ size_t need_of(const ts_linear_args *a, const Plan &pl) {
 // Small products that would be split anyway stay with lanes.hip, whose shorter start counts
 // there: 16 rows by bf16 128 x 4096 7.5 against 8.2 us, 30 by bf16 1024 x 2048 7.6 against 7.9,
 // 5 f32 rows by e4m3 1024 x 2048 8.0 against 8.4 (from 6 MB of f32 rows on 8.8 against 8.3).
-bool stream_fits(const ts_linear_args *a) {
+bool stream_always(const ts_linear_args *a) {
     if (!fits(a)) return false;
     if (block_form(a->w_dtype) || pair_of(a) || (a->stages & TS_BEFORE_RMS_NORM)) return true;
-    const uint64_t bytes = (uint64_t)a->n * a->k * (a->w_dtype == TS_E4M3 ? 1 : 2);
-    return bytes > (a->x_dtype == TS_F32 ? 4u << 20 : 8u << 20) || plan(a).splits == 1;
+    return (uint64_t)a->n * a->k * (a->w_dtype == TS_E4M3 ? 1 : 2) > (a->x_dtype == TS_F32 ? 4u << 20 : 8u << 20);
 }
 
-size_t stream_workspace(const ts_linear_args *a) { return need_of(a, plan(a)); }
+bool stream_fits(const ts_linear_args *a) { return stream_always(a) || (fits(a) && plan(a).splits == 1); }
+
+size_t stream_workspace(const ts_linear_args *a) {
+    const Plan pl = plan(a);
+    return pl.splits > 1 ? pl.splits * split_bytes(a) : 0;
+}
 
 int stream_launch(const ts_linear_args *a, void *stream) {
     StreamParams p;
@@ -675,10 +685,12 @@ int stream_launch(const ts_linear_args *a, void *stream) {
     p.m = a->m; p.n = a->n; p.k = a->k; p.stages = a->stages; p.out_bf16 = a->out_dtype == TS_BF16;
     int rc = linear_after(a, "lanes", &p.after);
     if (rc) return rc;
-    const Plan pl = plan(a);
-    const size_t need = need_of(a, pl);
-    const bool split = need && a->workspace && a->workspace_bytes >= need && aligned(a->workspace, 16);
-    p.splits = split ? pl.splits : 1;
+    // A workspace of fewer splits than the query names (sized for other row counts) gives the
+    // best plan of those, none the best unsplit one.
+    const size_t holds = a->workspace && aligned(a->workspace, 16) ? a->workspace_bytes / split_bytes(a) : 0;
+    const Plan pl = plan(a, (uint32_t)std::max<size_t>(1, std::min<size_t>(holds, kMostSplits)));
+    const bool split = pl.splits > 1;
+    p.splits = pl.splits;
     p.part = split ? (float *)a->workspace : nullptr;
     p.sumsq = split ? p.part + (size_t)pl.splits * a->m * a->n * (pair_of(a) ? 2 : 1) : nullptr;
     hipError_t e = pl.c.ready();

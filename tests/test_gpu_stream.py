@@ -76,3 +76,33 @@ def test_stream_without_workspace():
     abi.call("tessera_hip_linear", C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream))
     xn = O.rms_norm(xf, g, 1e-6)
     assert np.all(np.abs(from_dev(out) - xn.astype(np.float64) @ wf.T) <= 2 * linear_bound(xn, wf))
+
+
+@pytest.mark.parametrize("m,n,k,norm,silu", [(12, 256, 4096, True, False), (12, 130, 4096, True, True),
+                                             (40, 1000, 8192, False, False)])
+def test_stream_smaller_workspace(m, n, k, norm, silu):
+    """A workspace of fewer splits than the query names holds that many: the same product, and
+    nothing behind it is written."""
+    from tessera_amd import abi, rules as R
+    r = rng(m + n)
+    xd, wd, _, xf, wf, _ = operands(r, m, 2 * n if silu else n, k, "f32", "bf16")
+    gd = torch.ones(k, device="cuda") if norm else None
+    xn = O.rms_norm(xf, np.ones(k, np.float32), 1e-6) if norm else xf
+    want, bound = xn.astype(np.float64) @ wf.T.astype(np.float64), 2 * linear_bound(xn, wf)
+    if silu:
+        g, u, bg, bu = want[:, :n], want[:, n:], bound[:, :n], bound[:, n:]
+        want, bound = g / (1 + np.exp(-g)) * u, 1.1 * bg * np.abs(u) + np.abs(g) * bu + 1e-5
+    out = torch.empty((m, n), device="cuda")
+    stages = (abi.TS_BEFORE_RMS_NORM if norm else 0) | (abi.TS_AFTER_SILU_MUL if silu else 0)
+    a = R.linear_args(xd, wd, out, gain=gd, stages=stages)
+    need = abi.load().tessera_hip_linear_workspace(C.byref(a))
+    one = (m * n * (2 if silu else 1) + (m if norm else 0)) * 4
+    splits = need // one
+    assert splits >= 3 and need == splits * one
+    for size in (need, need - 1, 2 * one, 2 * one - 1, one, 1):
+        buf = torch.full((need + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        out.zero_()
+        a.workspace, a.workspace_bytes = buf.data_ptr(), size
+        abi.call("tessera_hip_linear", C.byref(a), R._stream())
+        assert np.all(np.abs(from_dev(out) - want) <= bound), f"{size} of {need} bytes"
+        assert bool((buf[size:] == 0xA5).all())
