@@ -134,18 +134,27 @@ typedef struct {
 } ts_linear_args;
 
 /* Picks `lanes` for m <= 64 and `tiled` otherwise (the cost select of
- * engine/plan/lower/src/cost.rs between the two rules). Where the tiles alone leave CUs
- * idle, k is split across groups with the workspace that the query names; without it the
- * product runs unsplit. */
+ * engine/plan/lower/src/cost.rs between the two rules). Where the columns or tiles alone leave
+ * CUs idle, k is split across groups, their sums in the workspace and added in split order
+ * (deterministic).
+ *  - The workspace query is for its m: a caller of several row counts takes the largest, which
+ *    is not always that of the most rows.
+ *  - A smaller workspace or none: past 64 rows k is not split; at 5..64 rows it is split as
+ *    often as the workspace holds, but TS_ERR_WORKSPACE for products that `lanes` does not
+ *    stream (below).
+ *  - How k is split follows from m, n, k, the types and the workspace, so the last bits of a
+ *    row's sums can differ with the number of rows beside it. */
 int tessera_hip_linear(const ts_linear_args *a, void *stream);
 size_t tessera_hip_linear_workspace(const ts_linear_args *a);
 
 /* Few rows (m <= 64): m <= 4 on the vector ALU (a wave streams whole weight
  * rows; block-form weights decode there too, bit-identical to the reference's
- * Block::dot, engine/ir/mem/src/block.rs:202-219); 5..64 on the matrix unit: a wave per 16 output columns, x staged once
- * per group in LDS, weights streamed once with 64-byte runs per lane, k split
- * across groups when the columns alone do not cover the chip (partials in the
- * workspace, summed in split order by a second kernel: deterministic).
+ * Block::dot, engine/ir/mem/src/block.rs:202-219); 5..64 on the matrix unit. There a wave
+ * streams 32 weight rows through LDS in units of k (64 values of bf16 weights, 128 of e4m3 and
+ * block forms), x staged once per group as matrix operands, k split across groups when the
+ * columns alone do not cover the chip (see tessera_hip_linear). Any other k, and small bf16 and
+ * e4m3 weights that would be split (up to 8 MiB, 4 MiB under f32 rows; no pair, no norm), run a
+ * wave per 16 output columns; those that are split refuse a workspace too small.
  * TS_BEFORE_RMS_NORM needs f32 x and m <= 16.
  * Replaces: rule "lanes" (engine/rules/linear/src/lanes.rs:17-143) and "thin"
  * (engine/rules/linear/src/thin.rs:11-104). */

@@ -139,7 +139,8 @@ def pack_f32(w):
 
 
 def linear(x, w, **kw):
-    """tiled or lanes by row count (the cost select between the two rules)."""
+    """tiled or lanes by row count (the cost select between the two rules). k is split by the row
+    count too: the last bits of a row's sums can differ with the number of rows beside it."""
     return _linear("tessera_hip_linear", x, w, **kw)
 
 
@@ -222,7 +223,9 @@ def moe_layer(h, router, w_in, w_out, *, top=8, shared_in=None, shared_out=None,
     scores = h . router^T; ids = top_k(scores); gates = softmax(take(scores, ids));
     inner = silu(h . gate_e) * (h . up_e) per pick; y = mix(inner . out_e, gates);
     plus the shared expert's SwiGLU when given. `scores` given: the router product is
-    skipped (router may be None). Returns (y, ids, gates)."""
+    skipped (router may be None). The last bits of a token's scores can differ with the number
+    of tokens (linear splits k by the row count), so near ties may pick another expert.
+    Returns (y, ids, gates)."""
     tokens = h.shape[0]
     if scores is None:
         scores = linear(h, router)
