@@ -306,9 +306,9 @@ __global__ __launch_bounds__(kThreads) void tiled_kernel(TiledParams p) {
 
 // ---------------------------------------------------------------------------
 // The pipelined form (k a multiple of 64): TM x TN tiles, 4 waves, and NS LDS stages KD
-// deep filled straight from memory with global_load_lds_dwordx4 (no staging registers,
+// deep filled straight from memory by 16-byte buffer loads to LDS (no staging registers,
 // no LDS stores), NS - 1 of them in flight ahead of the MFMAs, groups in an XCD-aware
-// order, and each configuration sized so two groups share a CU: one group's loads,
+// order, and each configuration sized so two groups (one form: three) share a CU: one group's loads,
 // barriers and epilogue overlap the other's matrix work. bf16 results leave through LDS
 // as whole rows.
 //  * bf16 rows and weights: waves in 2 x 2, each (TM/2) x (TN/2).
@@ -420,11 +420,18 @@ template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PI
 TS_DEV void pipe_tile(const TiledParams &p, char *lds, uint32_t n0, uint32_t m0, uint32_t mend, const char *w,
                       const uint16_t *scale, uint32_t split);
 
+// Groups that share a CU, a wave of each a SIMD: two, three of the form whose stages leave LDS
+// for them (bf16 rows by e4m3 on 64 x 64, 48 KiB: 700 rows by 4096 x 1024 11.7 -> 10.7 us, 704
+// tiles in one round; up to 512 tiles the same).
+template <int TM, int TN, int KD, int NS, bool XF32, bool W8, Ends END>
+constexpr int kShare = 3 * Pipe<TM, TN, KD, NS, XF32, W8>::LDS <= 160 * 1024 && TM * TN == 64 * 64 && END != kChain ? 3 : 2;
+
 // FEW (picked products): the matrices of at most p.few_most rows run as 32-row tiles. ROLL: the
 // steps are unrolled (not in a FEW kernel, whose two forms share the instruction cache).
 template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END, bool FEW>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void tiled_pipe_kernel(TiledParams p) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: two groups share a CU
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
+    kShare<TM, TN, KD, NS, XF32, W8, END>, kShare<TM, TN, KD, NS, XF32, W8, END>))) void tiled_pipe_kernel(TiledParams p) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];  // the only LDS: groups share a CU
     constexpr uint32_t OC = SILU ? TN / 2 : TN;  // output columns per tile
     uint32_t tx = blockIdx.x, ty = blockIdx.y, split = 0;
     if (!PICK) {
