@@ -757,7 +757,9 @@ TS_DEV void att_role(const DecodeStepArgs &p, Ctx &c, const Hand &hd, uint32_t h
                 float bm = sc[0];
 #pragma unroll
                 for (int i = 1; i < kPre; i++) bm = fmaxf(bm, sc[i]);
-                const float mn = fmaxf(m, rows4_max(bm));  // finite: key 4 wave <= pos
+                // -inf only where the wave has no key up to pos (pos < 4 wave): no ok then, so
+                // neither alpha nor a pk takes the difference of two -inf.
+                const float mn = fmaxf(m, rows4_max(bm));
                 const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
                 float acc[8], sum = 0.0f;
 #pragma unroll
