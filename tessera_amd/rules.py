@@ -26,9 +26,14 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# torch's own call for a raw stream handle, without the Stream object around it; not public.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-    # The handle of torch.cuda.current_stream(), without the Stream object around it.
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 class Workspace:

@@ -58,6 +58,16 @@ def test_calls_in_flight_do_not_share_scratch(op, monkeypatch):
     assert a + na <= b
 
 
+def test_stream_handle_without_the_raw_call(monkeypatch):
+    """A torch without its non-public call for the raw handle: the public one."""
+    from types import SimpleNamespace
+
+    from tessera_amd import rules as R
+    monkeypatch.setattr(R, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=1234))
+    assert R._stream() == 1234
+
+
 @pytest.mark.gpu
 def test_two_streams_match_serial_calls():
     """Expert products and decode attention enqueued on two streams at once give the bits that
