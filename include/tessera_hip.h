@@ -139,9 +139,8 @@ typedef struct {
  * (deterministic).
  *  - The workspace query is for its m: a caller of several row counts takes the largest, which
  *    is not always that of the most rows.
- *  - A smaller workspace or none: past 64 rows k is not split; at 5..64 rows it is split as
- *    often as the workspace holds, but TS_ERR_WORKSPACE for products that `lanes` does not
- *    stream (below).
+ *  - A smaller workspace or none: past 64 rows k is not split, at 5..64 rows it is split as
+ *    often as the workspace holds.
  *  - How k is split follows from m, n, k, the types and the workspace, so the last bits of a
  *    row's sums can differ with the number of rows beside it. */
 int tessera_hip_linear(const ts_linear_args *a, void *stream);
@@ -154,7 +153,7 @@ size_t tessera_hip_linear_workspace(const ts_linear_args *a);
  * block forms), x staged once per group as matrix operands, k split across groups when the
  * columns alone do not cover the chip (see tessera_hip_linear). Any other k, and small bf16 and
  * e4m3 weights that would be split (up to 8 MiB, 4 MiB under f32 rows; no pair, no norm), run a
- * wave per 16 output columns; those that are split refuse a workspace too small.
+ * wave per 16 output columns.
  * TS_BEFORE_RMS_NORM needs f32 x and m <= 16.
  * Replaces: rule "lanes" (engine/rules/linear/src/lanes.rs:17-143) and "thin"
  * (engine/rules/linear/src/thin.rs:11-104). */

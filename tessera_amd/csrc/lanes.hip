@@ -385,6 +385,11 @@ Plan plan(const ts_linear_args *a) {
     return pl;
 }
 
+// The sums of one split.
+size_t split_bytes(const ts_linear_args *a) {
+    return (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1) * sizeof(float);
+}
+
 using Kern = void (*)(LanesParams, float *);
 
 template <int MT, bool XF32, bool W8, bool CHAIN>
@@ -440,8 +445,8 @@ extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
     const size_t per = (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1);
     const size_t here = pl.splits <= 1 ? 0 : (size_t)pl.splits * per * sizeof(float);
     if (!ts::stream_fits(a)) return here;
-    // Fewer rows of a small product may run in this file, which refuses less than it needs and
-    // whose need grows with the rows: the size for the most rows serves them all.
+    // Fewer rows of a small product may run in this file, whose need grows with the rows: the size
+    // for the most rows serves them all.
     const size_t streamed = ts::stream_workspace(a);
     return ts::stream_always(a) ? streamed : std::max(here, streamed);
 }
@@ -463,10 +468,10 @@ extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
         return rc ? rc : ts::gemv_launch(a, stream);
     }
     if (ts::stream_fits(a)) return ts::stream_launch(a, stream);
-    const Plan pl = plan(a);
-    const size_t need = tessera_hip_lanes_workspace(a);
-    if (need && (!a->workspace || a->workspace_bytes < need))
-        return ts::fail(TS_ERR_WORKSPACE, "lanes: workspace %zu bytes, need %zu", a->workspace_bytes, need);
+    // A workspace of fewer splits than the query names holds that many.
+    Plan pl = plan(a);
+    const size_t holds = a->workspace && ts::aligned(a->workspace, 4) ? a->workspace_bytes / split_bytes(a) : 0;
+    pl.splits = (uint32_t)std::max<size_t>(1, std::min<size_t>(pl.splits, holds));
     LanesParams p;
     p.x = a->x; p.w = a->w; p.w_scale = (const uint16_t *)a->w_scale; p.gain = a->gain; p.a0 = a->a0;
     p.out = a->out; p.m = a->m; p.n = a->n; p.k = a->k; p.stages = a->stages; p.eps = a->eps;
@@ -482,7 +487,7 @@ extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
     Kern k = mt == 1 ? pick2<1>(xf, w8, silu, norm, chain)
            : mt == 2 ? pick2<2>(xf, w8, silu, norm, chain)
            : mt == 3 ? pick2<3>(xf, w8, silu, norm, chain) : pick2<4>(xf, w8, silu, norm, chain);
-    float *part = need ? (float *)a->workspace : nullptr;
+    float *part = pl.splits > 1 ? (float *)a->workspace : nullptr;
     hipLaunchKernelGGL(k, dim3(pl.groups, pl.splits), dim3(kWaves * 64), 0, (hipStream_t)stream, p, part);
     TS_CHECK_LAUNCH("lanes launch");
     if (pl.splits > 1) {

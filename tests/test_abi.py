@@ -162,20 +162,6 @@ def test_streamed_products_ask_for_what_they_write():
             assert lib.tessera_hip_lanes_workspace(C.byref(a)) <= most
 
 
-def test_small_split_products_refuse_a_missing_workspace():
-    """What the header says of products that are not streamed: refused before anything launches
-    (fake device addresses suffice) where their k is split, whatever the workspace lacks."""
-    lib = abi.load()
-    a = abi.LinearArgs()
-    a.x = a.w = a.out = 1 << 20
-    a.x_dtype = a.w_dtype = a.out_dtype = abi.TS_BF16
-    for a.m, a.n, a.k in ((16, 128, 4096), (8, 4096, 1032)):  # small weights; k in no whole units
-        need = lib.tessera_hip_linear_workspace(C.byref(a))
-        assert need > 0
-        for a.workspace, a.workspace_bytes in ((None, 0), (1 << 21, need - 1)):
-            assert lib.tessera_hip_linear(C.byref(a), None) == abi.TS_ERR_WORKSPACE
-
-
 def test_attend_step_refuses_workspace_sized_for_attend_rows():
     """Past 2048 keys the fused step splits a span into more partitions than
     attend_rows does; a workspace that holds only attend_rows' partials is refused

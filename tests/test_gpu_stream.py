@@ -106,3 +106,28 @@ def test_stream_smaller_workspace(m, n, k, norm, silu):
         abi.call("tessera_hip_linear", C.byref(a), R._stream())
         assert np.all(np.abs(from_dev(out) - want) <= bound), f"{size} of {need} bytes"
         assert bool((buf[size:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("x,w", FORMS)
+@pytest.mark.parametrize("m,n,k,silu", [(16, 70, 4072, False), (40, 130, 2056, True), (64, 200, 1032, False)])
+def test_lanes_smaller_workspace(m, n, k, silu, x, w):
+    """The kernel for any k (here in no whole units), split as often as its workspace holds: the
+    same product, and nothing behind the workspace is written."""
+    from tessera_amd import abi, rules as R
+    r = rng(m + n)
+    xd, wd, sd, xf, wf, want = operands(r, m, 2 * n if silu else n, k, x, w)
+    bound = linear_bound(xf, wf)
+    if silu:
+        g, u, bg, bu = want[:, :n], want[:, n:], bound[:, :n], bound[:, n:]
+        want, bound = O.act("silu", g) * u, 1.1 * bg * np.abs(u) + np.abs(g) * bu + 1e-5
+    out = torch.empty((m, n), device="cuda")
+    a = R.linear_args(xd, wd, out, w_scale=sd, stages=abi.TS_AFTER_SILU_MUL if silu else 0)
+    need, one = abi.load().tessera_hip_linear_workspace(C.byref(a)), m * n * (2 if silu else 1) * 4
+    assert need >= 3 * one and need % one == 0
+    for size in (need, need - 1, 2 * one, 2 * one - 1, 0):
+        buf = torch.full((need + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        out.zero_()
+        a.workspace, a.workspace_bytes = buf.data_ptr() if size else None, size
+        abi.call("tessera_hip_linear", C.byref(a), R._stream())
+        assert np.all(np.abs(from_dev(out) - want) <= bound), f"{size} of {need} bytes"
+        assert bool((buf[size:] == 0xA5).all())
