@@ -151,9 +151,8 @@ size_t tessera_hip_linear_workspace(const ts_linear_args *a);
  * Block::dot, engine/ir/mem/src/block.rs:202-219); 5..64 on the matrix unit. There a wave
  * streams 32 weight rows through LDS in units of k (64 values of bf16 weights, 128 of e4m3 and
  * block forms), x staged once per group as matrix operands, k split across groups when the
- * columns alone do not cover the chip (see tessera_hip_linear). Any other k, and small bf16 and
- * e4m3 weights that would be split (up to 8 MiB, 4 MiB under f32 rows; no pair, no norm), run a
- * wave per 16 output columns.
+ * columns alone do not cover the chip (see tessera_hip_linear). Any other k, and small weights
+ * (up to 8 MiB) where it is the shorter way, run a wave per 16 output columns.
  * TS_BEFORE_RMS_NORM needs f32 x and m <= 16.
  * Replaces: rule "lanes" (engine/rules/linear/src/lanes.rs:17-143) and "thin"
  * (engine/rules/linear/src/thin.rs:11-104). */

@@ -57,11 +57,11 @@ int block_check(const ts_linear_args *a, const char *rule);
 int block_gemv_launch(const ts_linear_args *a, void *stream);
 int block_tiled_launch(const ts_linear_args *a, void *stream);
 
-// 5..64 rows, weights streamed (stream.hip), arguments already checked: whether a product is
-// for it (stream_always: with any other row count too), the workspace its k split takes (a
-// smaller one holds fewer splits, none leaves k unsplit), and the launch.
+// 5..64 rows, weights streamed (stream.hip), arguments already checked: whether a product may
+// run there and whether it should, the workspace its k split takes (a smaller one holds fewer
+// splits, none leaves k unsplit), and the launch.
 bool stream_fits(const ts_linear_args *a);
-bool stream_always(const ts_linear_args *a);
+bool stream_better(const ts_linear_args *a);
 size_t stream_workspace(const ts_linear_args *a);
 int stream_launch(const ts_linear_args *a, void *stream);
 

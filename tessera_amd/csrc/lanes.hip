@@ -440,15 +440,10 @@ int check(const ts_linear_args *a) {
 extern "C" size_t tessera_hip_lanes_workspace(const ts_linear_args *a) {
     if (a && (a->stages & TS_AFTER_ARGMAX)) return (size_t)a->m * 8;  // the keys
     if (!a || a->m <= 4 || a->m > 64) return 0;
-    if (ts::block_form(a->w_dtype)) return ts::stream_fits(a) ? ts::stream_workspace(a) : 0;
+    if (ts::stream_fits(a) && ts::stream_better(a)) return ts::stream_workspace(a);
+    if (ts::block_form(a->w_dtype)) return 0;
     const Plan pl = plan(a);
-    const size_t per = (size_t)a->m * a->n * ((a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS ? 2 : 1);
-    const size_t here = pl.splits <= 1 ? 0 : (size_t)pl.splits * per * sizeof(float);
-    if (!ts::stream_fits(a)) return here;
-    // Fewer rows of a small product may run in this file, whose need grows with the rows: the size
-    // for the most rows serves them all.
-    const size_t streamed = ts::stream_workspace(a);
-    return ts::stream_always(a) ? streamed : std::max(here, streamed);
+    return pl.splits <= 1 ? 0 : pl.splits * split_bytes(a);
 }
 
 extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
@@ -467,7 +462,7 @@ extern "C" int tessera_hip_lanes(const ts_linear_args *a, void *stream) {
         rc = ts::linear_after(a, "lanes", &c);
         return rc ? rc : ts::gemv_launch(a, stream);
     }
-    if (ts::stream_fits(a)) return ts::stream_launch(a, stream);
+    if (ts::stream_fits(a) && ts::stream_better(a)) return ts::stream_launch(a, stream);
     // A workspace of fewer splits than the query names holds that many.
     Plan pl = plan(a);
     const size_t holds = a->workspace && ts::aligned(a->workspace, 4) ? a->workspace_bytes / split_bytes(a) : 0;

@@ -527,6 +527,7 @@ struct Choice {
     hipError_t (*ready)();  // raises the kernel's dynamic LDS size, once
     int lds, cols, span, threads;  // dynamic LDS, output columns of a group, k of a step
     int work;                      // operands of x a wave multiplies in a step
+    int slices, tiles, parts;      // S, row tiles of 16, bf16 parts of x
 };
 
 template <int F, int MT, bool XF32, bool PAIR, int S, bool NORM>
@@ -541,7 +542,7 @@ template <int F, int MT, bool XF32, bool PAIR, int S, bool NORM = false>
 Choice choice() {
     using P = Shape<F, MT, XF32, PAIR, S>;
     return Choice{(const void *)stream_kernel<F, MT, XF32, PAIR, S, NORM>, ready<F, MT, XF32, PAIR, S, NORM>, P::LDS,
-                  P::OC, S * Unit<F>::UNIT, P::THREADS, Unit<F>::STEPS * MT * P::PARTS};
+                  P::OC, S * Unit<F>::UNIT, P::THREADS, Unit<F>::STEPS * MT * P::PARTS, S, MT, P::PARTS};
 }
 
 struct Plan {
@@ -550,15 +551,50 @@ struct Plan {
     float cost;
 };
 
+constexpr uint32_t kMostSplits = 32;
+
 bool pair_of(const ts_linear_args *a) { return (a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS; }
 
-// The k split of a choice: what takes the least time, in steps of a group (~0.6 us, more
-// where a step's matrix work outlasts its loads): rounds of resident groups, three steps to
-// fill each one's pipeline, and for a split the time of six for the second kernel and its
-// sums' way to memory and back (1.3 MB a step). Measured over S and
-// splits: 16 rows by bf16 4096 x 1536 7.7 us at S 4 unsplit, 8.8 at S 2 in 6 and S 1 in 8; 64
-// f32 rows by 2 x 3072 x 1024 14.1 us in 4 splits, 15.9 in 8; 16 by 2 x 1536 x 4096 11.7 at S
-// 4 in 4, 13.1 at S 1 in 16; 8 by e4m3 2 x 14336 x 4096 29.3 to 30.6 whichever.
+// Plain weights of up to this many bytes are small: what counts is latency, and lanes.hip may be
+// the shorter way.
+constexpr uint64_t kSmall = 8u << 20;
+
+bool small(const ts_linear_args *a) {
+    return !block_form(a->w_dtype) &&
+           (uint64_t)a->n * a->k * (pair_of(a) ? 2 : 1) * (a->w_dtype == TS_E4M3 ? 1 : 2) <= kSmall;
+}
+
+// What a choice takes with k split s ways, us: its start, the steps of each round of resident
+// groups, and for a split the second kernel and its sums. For block forms and small plain
+// weights, fits to products timed at every S and 1 to 16 splits (128 to 14336 weight rows of
+// 1024 to 8192, 8 to 64 rows, both row types, pairs, weights from HBM and from the caches; mean
+// error 2% for block forms, 8% for plain ones). What these choose takes 0.3% (block forms) and 1%
+// (plain) more than the best choice, where the rule of the large plain weights took 8% and
+// 7%: 48 bf16 rows by int4_g32 14336 x 2048 unsplit 30.7 us, in 4 splits 18.5; by bf16 1024 x
+// 2048 unsplit 12.0, in 8 splits 7.7.
+float took_us(const ts_linear_args *a, const Choice &c, uint32_t s, uint32_t resident) {
+    const bool block = block_form(a->w_dtype), pair = pair_of(a);
+    const uint32_t groups = (a->n + c.cols - 1) / c.cols * s, steps = (a->k + c.span - 1) / c.span, each = (steps + s - 1) / s;
+    const uint32_t rounds = (groups + resident - 1) / resident;
+    const float mt = (float)c.tiles, x = (float)(c.slices * c.tiles * c.parts), u = a->w_dtype == TS_E4M3 ? 2.0f : 1.0f;
+    const float step = block ? (c.slices == 2 ? 0.85f + 0.13f * x : 1.3f + 0.12f * x)
+                             : 0.4f + u * (0.027f * x + 0.025f * mt * c.parts + 0.031f * mt * (c.parts - 1));
+    float t = (block ? 2.5f + 0.55f * mt : 3.18f + 0.33f * mt + (c.tiles == 4 ? 0.16f : 0.0f)) + rounds * each * step +
+              (rounds - 1) * (block ? 1.0f : 0.92f);
+    if (s > 1) {
+        const float sums = 4e-6f * s * std::max(a->m, 16u) * a->n * (pair ? 2 : 1);
+        t += block ? 2.9f - 0.38f * mt + 0.55f * sums : 2.94f - 0.38f * mt + (pair ? 0.81f : 0.0f) + 0.62f * sums;
+    }
+    return t;
+}
+
+// The k split of a choice: what takes the least time. Large plain weights: in steps of a group
+// (~0.6 us, more where a step's matrix work outlasts its loads), rounds of resident groups,
+// three steps to fill each one's pipeline, and for a split the time of six for the second
+// kernel and its sums' way to memory and back (1.3 MB a step). Measured over S and splits: 16
+// rows by bf16 4096 x 1536 7.7 us at S 4 unsplit, 8.8 at S 2 in 6 and S 1 in 8; 64 f32 rows by
+// 2 x 3072 x 1024 14.1 us in 4 splits, 15.9 in 8; 16 by 2 x 1536 x 4096 11.7 at S 4 in 4, 13.1
+// at S 1 in 16; 8 by e4m3 2 x 14336 x 4096 29.3 to 30.6 whichever.
 Plan plan_splits(const ts_linear_args *a, const Choice &c, uint32_t most) {
     const uint32_t groups = (a->n + c.cols - 1) / c.cols, steps = (a->k + c.span - 1) / c.span;
     // Two waves a SIMD: one group of 8 a CU, two of 4 where their LDS allows. (Counted by LDS
@@ -567,10 +603,14 @@ Plan plan_splits(const ts_linear_args *a, const Choice &c, uint32_t most) {
     const uint32_t resident = kCus * std::min(8 * 64 / c.threads, kMaxLds / c.lds);
     const float sums = (float)a->m * a->n * (pair_of(a) ? 2 : 1) * sizeof(float);
     const float step = std::max(1.0f, c.work / 12.0f);
+    const bool block = block_form(a->w_dtype), us = block || small(a);
     Plan best = {c, 1, 1e30f};
-    for (uint32_t s = 1; s <= std::min(steps, most); s++) {
+    for (uint32_t s = 1; s <= std::min({steps, most, us && !block ? 16u : kMostSplits}); s++) {  // 16: the fit's range
+        // One step of little matrix work fills no pipeline.
+        if (us && !block && s > 1 && 2 * s > steps && c.tiles * c.parts < 4) break;
         const uint32_t rounds = (groups * s + resident - 1) / resident;
-        const float took = (float)(rounds * ((steps + s - 1) / s + 3)) * step + (s > 1 ? 6.0f + s * sums / 1.3e6f : 0.0f);
+        const float took = us ? took_us(a, c, s, resident)
+                              : (float)(rounds * ((steps + s - 1) / s + 3)) * step + (s > 1 ? 6.0f + s * sums / 1.3e6f : 0.0f);
         if (took < best.cost) {
             best.splits = s;
             best.cost = took;
@@ -628,8 +668,6 @@ Plan plan_rows(const ts_linear_args *a, uint32_t most) {
          : mt == 3 ? plan_of<F, 3>(a, most) : plan_of<F, 4>(a, most);
 }
 
-constexpr uint32_t kMostSplits = 32;
-
 // most: the splits that the workspace holds.
 Plan plan(const ts_linear_args *a, uint32_t most = kMostSplits) {
     switch (a->w_dtype) {
@@ -662,16 +700,22 @@ size_t split_bytes(const ts_linear_args *a) {
 
 }  // namespace
 
-// Small products that would be split anyway stay with lanes.hip, whose shorter start counts
-// there: 16 rows by bf16 128 x 4096 7.5 against 8.2 us, 30 by bf16 1024 x 2048 7.6 against 7.9,
-// 5 f32 rows by e4m3 1024 x 2048 8.0 against 8.4 (from 6 MB of f32 rows on 8.8 against 8.3).
-bool stream_always(const ts_linear_args *a) {
-    if (!fits(a)) return false;
-    if (block_form(a->w_dtype) || pair_of(a) || (a->stages & TS_BEFORE_RMS_NORM)) return true;
-    return (uint64_t)a->n * a->k * (a->w_dtype == TS_E4M3 ? 1 : 2) > (a->x_dtype == TS_F32 ? 4u << 20 : 8u << 20);
-}
+bool stream_fits(const ts_linear_args *a) { return fits(a); }
 
-bool stream_fits(const ts_linear_args *a) { return stream_always(a) || (fits(a) && plan(a).splits == 1); }
+// Small products go where the times say (a norm is cheaper here at any size, and lanes.hip takes
+// 1.7 times as long for a k that is no multiple of its 128): lanes.hip starts sooner and splits
+// finer, here a step takes less. lanes.hip's time is a fit to the same
+// products (mean error 4%). With weights from HBM, 64 bf16 rows by bf16 1024 x 1024 7.3 us
+// there, 11.4 here; 8 rows by 4096 x 1024 6.5 and 6.0, the pair 7.7 and 6.1; 8 by e4m3 2 x 1024
+// x 4096 7.8 and 9.5.
+bool stream_better(const ts_linear_args *a) {
+    if (!small(a) || (a->stages & TS_BEFORE_RMS_NORM) || a->k % 128) return true;
+    const float mt = (float)((a->m + 15) / 16), parts = a->x_dtype == TS_F32 ? 2.0f : 1.0f;
+    const float values = (float)a->n * a->k * (pair_of(a) ? 2 : 1) / 1048576.0f;
+    const float lanes = 4.7f + 0.54f * mt + 0.8f * mt * (parts - 1.0f) + (0.2f + 0.08f * mt * parts) * values +
+                        (pair_of(a) ? 1.23f : 0.0f) + (a->w_dtype == TS_E4M3 ? 0.0f : 0.52f);
+    return plan(a).cost < 0.97f * lanes;
+}
 
 size_t stream_workspace(const ts_linear_args *a) {
     const Plan pl = plan(a);
