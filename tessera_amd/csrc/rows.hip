@@ -329,7 +329,9 @@ extern "C" int tessera_hip_rms_norm(const ts_norm_args *a, void *stream) {
     TS_REQUIRE(x && gain && out, "rms_norm: null pointer");
     TS_REQUIRE(width >= 1, "rms_norm: width 0");
     if (rows == 0) return TS_OK;
-    if (width <= 4096) {  // wider rows would not fit the registers beside their gains
+    // Wider rows would not fit the registers beside their gains; one value a lane has nothing to
+    // keep in flight (4096 rows of 64 2.9 us in the loop, 3.1 in registers).
+    if (width > 64 && width <= 4096) {
         auto k = width <= 512 ? rms_norm_row_kernel<8> : width <= 1024 ? rms_norm_row_kernel<16>
                : width <= 2048 ? rms_norm_row_kernel<32> : rms_norm_row_kernel<64>;
         hipLaunchKernelGGL(k, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream, x, gain, out, rows, width, eps);
@@ -397,9 +399,12 @@ extern "C" int tessera_hip_qk_norm_rope_append(const ts_qk_args *a, void *stream
     p.rows = rows; p.heads = heads; p.kv_heads = kv_heads; p.keys = keys; p.kept_pages = kept_pages;
     p.page_shift = kept_table ? (uint32_t)__builtin_ctz(page) : 0;
     p.eps = eps; p.theta = theta;
-    // Few rows: a wave a head, so that more waves share the work than a group a row gives (8
-    // rows of 32 heads 3.0 against 5.1 us, 1000 rows 15.5 against 8.9).
-    if (rows < 256) {
+    // Few rows or few heads a row: a wave a head, so that more waves share the work than a group
+    // a row gives. 32 heads: 8 rows 3.0 against 5.1 us, 256 rows 5.9 and 5.7, 1000 rows 15.5
+    // and 8.9; 24 heads: 300 rows 5.0 and 5.4, 512 rows 7.1 and 5.9; 4 heads: 4096 rows 8.0
+    // and 10.4.
+    const uint32_t per_row = heads + 2 * kv_heads;
+    if (per_row < 16 || (uint64_t)rows * per_row < 8192) {
         const uint32_t waves = rows * (heads + 2 * kv_heads);
         hipLaunchKernelGGL(qk_norm_rope_append_kernel, dim3((waves + 3) / 4), dim3(256), 0, (hipStream_t)stream, p);
     } else {

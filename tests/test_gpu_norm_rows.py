@@ -52,3 +52,28 @@ def test_qk_norm_rope_append_many_rows(heads, kvh):
 
     for a, b in zip(call([(0, rows)]), call([(0, 150), (150, rows)])):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("heads,kvh,rows", [(12, 2, 512), (7, 7, 391), (10, 2, 600), (8, 4, 1200)])
+def test_qk_norm_rope_append_group_a_row(heads, kvh, rows):
+    """Around the rule of the two forms (16 heads a row, 8192 heads in all): every row's bits are
+    those it has among few rows, which take a wave a head."""
+    from tessera_amd import rules as R
+    r = rng(rows)
+    qkv = to_dev(r.standard_normal((rows, (heads + 2 * kvh) * 128)).astype(np.float32), torch)
+    qg, kg = (to_dev((1 + 0.02 * r.standard_normal(128)).astype(np.float32), torch) for _ in range(2))
+    pos = to_dev(r.permutation(rows).astype(np.uint32), torch, torch.int32)
+    slots = torch.zeros(rows, dtype=torch.int32, device="cuda")
+
+    def call(step):
+        q = torch.full((rows, heads, 128), 7.0, device="cuda")
+        k = torch.zeros((rows, kvh, 128), dtype=torch.bfloat16, device="cuda")
+        v = torch.zeros_like(k)
+        for lo in range(0, rows, step):
+            s = slice(lo, min(lo + step, rows))
+            R.qk_norm_rope_append(qkv[s], qg, kg, q[s], k, v, slots[s], pos[s], heads=heads, kv_heads=kvh, keys=rows,
+                                  eps=1e-6, theta=1e6)
+        return q, k, v
+
+    for a, b in zip(call(rows), call(100)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
