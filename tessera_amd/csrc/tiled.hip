@@ -427,7 +427,9 @@ template <int TM, int TN, int KD, int NS, bool XF32, bool W8, Ends END>
 constexpr int kShare = 3 * Pipe<TM, TN, KD, NS, XF32, W8>::LDS <= 160 * 1024 && TM * TN == 64 * 64 && END != kChain ? 3 : 2;
 
 // FEW (picked products): the matrices of at most p.few_most rows run as 32-row tiles. ROLL: the
-// steps are unrolled (not in a FEW kernel, whose two forms share the instruction cache).
+// steps are unrolled (not in a FEW kernel, whose two forms share the instruction cache, nor in
+// 32-row tiles, where f32 rows by e4m3 got slower: 64 rows on 64 matrices of 2 x 1024 x 2048 57 -> 60
+// us).
 template <int TM, int TN, int KD, int NS, bool XF32, bool W8, bool SILU, bool PICK, Ends END, bool FEW>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
     kShare<TM, TN, KD, NS, XF32, W8, END>, kShare<TM, TN, KD, NS, XF32, W8, END>))) void tiled_pipe_kernel(TiledParams p) {
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
                     p, lds, n0, p.row_start[e] + (y - p.tile_start[e]) * 32, mend, w, scale, split);
         m0 = p.row_start[e] + (y - p.tile_start[e]) * TM;
     }
-    pipe_tile<TM, TN, KD, NS, XF32, W8, SILU, PICK, END, !FEW>(p, lds, n0, m0, mend, w, scale, split);
+    pipe_tile<TM, TN, KD, NS, XF32, W8, SILU, PICK, END, !FEW && TM != 32>(p, lds, n0, m0, mend, w, scale, split);
 }
 
 // The tile of rows [m0, min(m0 + TM, mend)) and of the columns from n0 on.
@@ -867,14 +869,21 @@ int pipe_small(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) 
               : pipe_launch<64, 64, 64, 4, false, false, false, END>(p, silu, stream);
 }
 
-// 128 x 128 tiles. FEW: 32 x 128 for the matrices of few rows, the four waves side by side
-// along the columns.
+// 128 x 128 tiles. FEW: 32 x 128 for the matrices of few rows.
 template <bool PICK, Ends END = kPlain, bool FEW = false>
 int pipe_wide(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
     if (xf) return w8 ? pipe_launch<128, 128, 64, 2, true, true, PICK, END, FEW>(p, silu, stream)
                       : pipe_launch<128, 128, 32, 3, true, false, PICK, END, FEW>(p, silu, stream);
     return w8 ? pipe_launch<128, 128, 64, 3, false, true, PICK, END, FEW>(p, silu, stream)
               : pipe_launch<128, 128, 64, 2, false, false, PICK, END, FEW>(p, silu, stream);
+}
+
+// 32 x 128 tiles alone: the four waves side by side along the columns.
+int pipe_few(const TiledParams &p, bool xf, bool w8, bool silu, void *stream) {
+    if (xf) return w8 ? pipe_launch<32, 128, 64, kFewStages<true>, true, true, true>(p, silu, stream)
+                      : pipe_launch<32, 128, 64, kFewStages<true>, true, false, true>(p, silu, stream);
+    return w8 ? pipe_launch<32, 128, 64, kFewStages<false>, false, true, true>(p, silu, stream)
+              : pipe_launch<32, 128, 64, kFewStages<false>, false, false, true>(p, silu, stream);
 }
 
 using Kern = void (*)(TiledParams);
@@ -1064,10 +1073,11 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // on 4 matrices 67 -> 46 us, 2 x 1536 x 4096 102 -> 74; on Zipf-distributed matrices within 2%
     // of 32-row tiles alone).
     const uint32_t pick_gx = a->stages & TS_AFTER_SILU_MUL ? (a->n + 63) / 64 : (a->n + 127) / 128;
-    const bool few = pipe && a->rows <= 16ull * a->count;
-    const uint32_t few_most = !few ? 0 : (uint64_t)a->rows * pick_gx > 32 * 1024 ? 64 : 0xffffffffu;
+    const bool few = pipe && a->rows <= 16ull * a->count, mixed = few && (uint64_t)a->rows * pick_gx > 32 * 1024;
+    const uint32_t few_most = mixed ? 64 : 0;
     ts::Route route;
-    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, BM, few_most, a->workspace, &route, stream);
+    int rc = ts::route_launch(a->ids, a->rows, a->first, a->count, few && !mixed ? 32 : BM, few_most, a->workspace, &route,
+                              stream);
     if (rc) return rc;
     const bool silu = a->stages & TS_AFTER_SILU_MUL;
     TiledParams p;
@@ -1089,7 +1099,7 @@ extern "C" int tessera_hip_picked(const ts_picked_args *a, void *stream) {
     // A stage chain takes the register-staged kernel (the pipelined one's chain variant spills).
     // 128 x 192 tiles where the columns divide evenly (fewer re-reads of the gathered
     // rows per weight byte: C5 gate/up 1249 -> 1202 us), else 128 x 128.
-    if (few) return pipe_wide<true, kPlain, true>(p, xf, w8, silu, stream);
+    if (few) return mixed ? pipe_wide<true, kPlain, true>(p, xf, w8, silu, stream) : pipe_few(p, xf, w8, silu, stream);
     if (pipe) {
         if (!xf && !w8 && (silu ? a->n % 96 : a->n % 192) == 0)
             return pipe_launch<128, 192, 64, 2, false, false, true>(p, silu, stream);
