@@ -559,10 +559,11 @@ bool pair_of(const ts_linear_args *a) { return (a->stages & TS_AFTER_SILU_MUL) |
 // the shorter way.
 constexpr uint64_t kSmall = 8u << 20;
 
-bool small(const ts_linear_args *a) {
-    return !block_form(a->w_dtype) &&
-           (uint64_t)a->n * a->k * (pair_of(a) ? 2 : 1) * (a->w_dtype == TS_E4M3 ? 1 : 2) <= kSmall;
+uint64_t plain_bytes(const ts_linear_args *a) {
+    return (uint64_t)a->n * a->k * (pair_of(a) ? 2 : 1) * (a->w_dtype == TS_E4M3 ? 1 : 2);
 }
+
+bool small(const ts_linear_args *a) { return !block_form(a->w_dtype) && plain_bytes(a) <= kSmall; }
 
 // What a choice takes with k split s ways, us: its start, the steps of each round of resident
 // groups, and for a split the second kernel and its sums. For block forms and small plain
@@ -709,7 +710,15 @@ bool stream_fits(const ts_linear_args *a) { return fits(a); }
 // there, 11.4 here; 8 rows by 4096 x 1024 6.5 and 6.0, the pair 7.7 and 6.1; 8 by e4m3 2 x 1024
 // x 4096 7.8 and 9.5.
 bool stream_better(const ts_linear_args *a) {
-    if (!small(a) || (a->stages & TS_BEFORE_RMS_NORM) || a->k % 128) return true;
+    if (block_form(a->w_dtype) || (a->stages & TS_BEFORE_RMS_NORM) || a->k % 128) return true;
+    // Up to twice that, up to 16 bf16 rows by pairs of bf16 weights that are split here: from HBM,
+    // where a model's weights are, 8 rows by 2 x 1024 x 4096 take 8.8 us there and 10.1 here (from
+    // the caches 7.9 both), by 2 x 512 x 8192 10.0 and 11.4 (9.0 and 8.4). Single weights are
+    // faster here from the caches by more than they lose from HBM (2048 x 4096 6.4 against 7.6, 9.4
+    // against 8.6), f32 rows, e4m3 and more rows either way.
+    if (!small(a))
+        return a->m > 16 || a->x_dtype == TS_F32 || a->w_dtype == TS_E4M3 || !pair_of(a) || plain_bytes(a) > 2 * kSmall ||
+               plan(a).splits == 1;
     const float mt = (float)((a->m + 15) / 16), parts = a->x_dtype == TS_F32 ? 2.0f : 1.0f;
     const float values = (float)a->n * a->k * (pair_of(a) ? 2 : 1) / 1048576.0f;
     const float lanes = 4.7f + 0.54f * mt + 0.8f * mt * (parts - 1.0f) + (0.2f + 0.08f * mt * parts) * values +
