@@ -906,12 +906,14 @@ namespace {
 
 // The k split of a product of more than 64 rows whose tiles alone leave CUs idle: times in us,
 // from what the pipelined tiles take a 64-deep step with one group a CU and with two (64 x 64
-// 0.19 and 0.35, f32 rows 0.38 and 0.62; 128 x 128 0.58 and 0.85, e4m3 0.51, f32 rows 1.0 and
-// 1.7; past two in proportion) and what the second kernel takes (4.5 us and 0.35 a MB of sums).
-// Measured, unsplit against split, over 880 products of 65 to 2048 rows by 128 to 4096 x 1024 to
-// 14336: what this chooses takes 0.1% more than the better one in the mean, at most 9%. 128 f32
-// rows by 1024 x 3072 23.8 -> 11.6 us, 1200 by 2048 x 8192 129 -> 91; 200 bf16 rows by 4096 x
-// 4096 15.8 unsplit, 21.1 in four splits.
+// 0.21 and 0.33, e4m3 0.2, f32 rows 0.4 and 0.62; 128 x 128 0.65 and 0.82, e4m3 0.49, f32 rows
+// 0.99 and 1.7; past two in proportion) and what the second kernel takes (3.2, 0.1 a split and
+// 0.37 a MB of sums). Fitted to every split of 980 products of 65 to 2048 rows by 128 to 8192 x
+// 1024 to 14336 with weights in the caches and from HBM, between which the prices stand: what this
+// chooses takes 0.5% more than the best split in the mean, 18% at most (128 bf16 rows by 2048 x
+// 2048 from HBM). 128 f32 rows by 1024 x 3072 23.8 -> 11.6 us, 1200 by 2048 x 8192 129 -> 91; 300
+// bf16 rows by e4m3 2560 x 9728 32.0 -> 28.0, from HBM 36.1 -> 31.0; 200 by bf16 4096 x 4096 15.8
+// unsplit, 21.1 in four splits.
 struct Split {
     uint32_t splits;
     bool wide;  // 128 x 128 tiles
@@ -920,21 +922,22 @@ struct Split {
 constexpr uint64_t kCus = 256;
 
 Split plan_split(const ts_linear_args *a) {
-    const bool pair = (a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS, xf = a->x_dtype == TS_F32;
+    const bool pair = (a->stages & TS_AFTER_SILU_MUL) || a->w_dtype == TS_F32_PARTS;
+    const bool xf = a->x_dtype == TS_F32, w8 = a->w_dtype == TS_E4M3;
     const uint32_t steps = a->k / 64;
     Split best = {1, false};
     auto tiles = [&](uint32_t t) { return (uint64_t)((a->n + (pair ? t / 2 : t) - 1) / (pair ? t / 2 : t)) * ((a->m + t - 1) / t); };
     const float sums = 4e-6f * (float)a->m * (float)a->n * (pair ? 2 : 1);  // MB
     auto step_us = [&](bool wide, uint64_t groups) {
-        if (groups <= kCus) return wide ? (xf ? 1.02f : a->w_dtype == TS_E4M3 ? 0.51f : 0.58f) : xf ? 0.38f : 0.19f;
-        const float two = wide ? (xf ? 1.7f : 0.85f) : xf ? 0.62f : 0.35f;
+        if (groups <= kCus) return wide ? (xf ? 0.99f : w8 ? 0.49f : 0.65f) : xf ? 0.4f : w8 ? 0.2f : 0.21f;
+        const float two = wide ? (xf ? 1.7f : 0.82f) : xf ? 0.62f : 0.33f;
         return two / 2 * (float)((groups + kCus - 1) / kCus);
     };
     auto cost = [&](bool wide, uint32_t s) {
-        return (float)((steps + s - 1) / s) * step_us(wide, tiles(wide ? 128 : 64) * s) + (s > 1 ? 4.5f + 0.35f * s * sums : 0.0f);
+        return (float)((steps + s - 1) / s) * step_us(wide, tiles(wide ? 128 : 64) * s) + (s > 1 ? 3.2f + s * (0.1f + 0.37f * sums) : 0.0f);
     };
     if (tiles(64) > 1024) return best;  // enough tiles of some size
-    float least = 0.94f * cost(tiles(128) >= 256, 1);
+    float least = cost(tiles(128) >= 256, 1);
     for (int wide = 0; wide < 2; wide++)
         for (uint32_t s = 2; s <= 16 && 4 * s <= steps; s++)
             if (cost(wide, s) < least) {
